@@ -2,30 +2,44 @@
 // the gfx950 matrix cores.
 //
 // Same results as the grouped dot-product kernels of k_moe.hip, bit for bit:
-// the integer group sums I_g = sum (q - zp) * qs are formed by
-// v_mfma_f32_32x32x16_f16 on operands that hold small integers exactly, and
-// the float epilogue is the canonical chain of the Q8_K path
+// the integer group sums I_g = sum (q - zp) * qs are formed exactly by the
+// matrix cores, and the float epilogue is the canonical chain of the Q8_K path
 //   blk = fma(s3,I3, fma(s2,I2, fma(s1,I1, fma(s0,I0,0))));  acc = fma(d_b, blk, acc)
 // (sf37_cuda.cu:4226-4274 sums the same integers; this build fixes the order).
 //
-// Exactness.  A weight code pair is turned into one dword of two fp16 values
-// with a mask and an add: the codes sit in the mantissas under a fixed
-// exponent, so each half equals  B + (q - zp)  for a power-of-two bias B that
-// depends only on the element's position (fp16 exponent 25 - p for a code at
-// mantissa bit p).  Activation codes qs are int8, exact in fp16.  The MFMA
-// accumulator starts at  C = -sum_e B_e * qs_e  (a per-token, per-group
-// integer the activation kernel precomputes), so it ends at exactly I_g; all
-// partial sums are integers below 2^24 in magnitude, hence exact in fp32 in
-// any summation order.
+// Exactness.  The operands are 6-bit floats (v_mfma_f32_32x32x64_f8f6f4), one
+// MFMA instruction spanning one 64-group.  A 3- or 2-bit weight code in the
+// low bits of an E2M3 field is that code times 1/8 (E2M3 is linear up to
+// 15/8), so dequantising is a mask per dword.  An activation code |qs| <= 128
+// is split as qs = 16 h + l with the sign of qs on both: l (0..15) is linear
+// in E2M3 (l/8), h (0..8) is exact in E3M2 as 2h.  The two MFMAs of a group
+// add 2h * q/8 and l/8 * q/8, together q * qs / 64, and a third one (fp16,
+// K = 8) starts the accumulator at -zp * gsum / 64, gsum = sum qs cut into
+// two exact fp16 parts.  Every partial sum is a multiple of 1/64 below
+// 2^18, exact in fp32 in any order, so D = I_g / 64, and fma(64 s_g, D, blk)
+// rounds the same value as fma(s_g, I_g, blk).
+//
+// Why 6 bits: measured per SIMD (four waves, ns), a 64-group of a 32 x 32
+// tile takes 65 as four fp16 32x32x16 MFMAs and 51 as these three, and the
+// time of the VALU operations adds to it (about 1 ns each, hardly any
+// overlap), so what counts is the sum: the fp16 operands took 1.5 VALU
+// operations per weight code to dequantise, these 0.3-0.4.  Gate/up and down
+// at 4096 tokens: 1153 + 626 us with fp16 operands, 885 + 495 now; 187 tokens
+// (groups of ~5 pairs) 491 + 220 -> 336 + 142 us.  What bounds them: at 4096
+// tokens about half of the time is MFMA and VALU issue, the rest waits for
+// loads: a weight load touches all 32 rows of its lanes, so the address units
+// are ~70 % busy (no weight loads: 700 us; weights through LDS tiles by
+// direct loads, whole runs of a row at a time: 1020 us, the words' LDS reads
+// cost more than that saves).
 //
 // Layouts.  Activations are re-quantised to Q8_K (sf37_cuda.cu:4168-4205,
-// bit-exact) and written as fp16 codes in the MFMA lane order of the weight
-// format, plus a table per (row, 256-block): C of the four 64-groups and d.
-// A workgroup owns (tile of <= 128 pairs of one expert, row tile); it stages
-// the tile's activation blocks in LDS by direct global->LDS loads (two
-// buffers, one block ahead) and each wave streams its own weight rows into
-// registers one block ahead, dequantises them in registers and runs the
-// MFMAs: 4 token blocks x one 32-column weight block per wave.
+// bit-exact) and written per (row, 256-block) as 384 bytes of 6-bit fields
+// (24 16-byte pieces in the order the LDS reads want, below), the four
+// groups' -gsum/64 as fp16 pairs and the scale d.  A workgroup owns (tile of
+// <= 64 pairs of one expert, row tile); it stages the tile's blocks in LDS by
+// direct global->LDS loads (two buffers, one block ahead), each wave loads
+// its own weight rows into registers one block ahead, dequantises a block at
+// once (24 registers) and runs the MFMAs over the tile's 32-pair blocks.
 #include <type_traits>
 
 #include "sf37_blocks.h"
@@ -33,38 +47,26 @@
 
 namespace {
 
-typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+typedef _Float16 h4v __attribute__((ext_vector_type(4)));
 typedef float f16v __attribute__((ext_vector_type(16)));
 
 constexpr uint32_t PF_T = 64;           // pairs per tile
-constexpr uint32_t PF_TB = PF_T / 32u;  // 32-pair MFMA blocks per tile
-// Waves per workgroup (32 weight columns each) and activation buffers:
-// gate/up one 8-wave workgroup per CU (two waves per SIMD), activations
-// three buffers deep; down two 4-wave workgroups per CU (their barriers do
-// not stall each other's SIMDs), two buffers.  Measured: 4-wave down
-// workgroups 649 against 696 us at 4096 tokens; 4-wave gate/up 1307
-// against 1263 us.
-template <bool Q3> struct pf_cfg {
-    static constexpr uint32_t NW = Q3 ? 8u : 4u;
-    static constexpr uint32_t NBUF = Q3 ? 3u : 2u;
-    static constexpr uint32_t ROWS = (Q3 ? 16u : 32u) * NW;   // F rows (gate/up) or output rows per workgroup
-};
-constexpr uint32_t PF_GU_R = pf_cfg<true>::ROWS;    // 128
-constexpr uint32_t PF_DN_R = pf_cfg<false>::ROWS;   // 128
-constexpr uint32_t PF_CD_ROWS = 8;                  // table rows of LDS per buffer (5 used)
-constexpr uint32_t PF_TAB = 8;          // floats per (row, block) table entry: C0..C3, d
-// pf_expert table loads (dword): one row of PF_T floats per load, at row
-// index wave (8 waves, wave <= 7) or max(wave, 4) (4 waves).
-static_assert(PF_T * 4u == 256u, "a table load (64 dwords) writes exactly one row");
-static_assert(pf_cfg<true>::NW <= PF_CD_ROWS && pf_cfg<false>::NW <= PF_CD_ROWS && 4u < PF_CD_ROWS,
-              "pf_expert table rows stay in their buffer");
-// LDS layout of one activation block: 4 groups of 32 tile slots; in a group
-// slot t (0..31) starts at PF_RS * (t % 16) + 512 * (t / 16), so one 64-lane
-// load fills slots t and t + 16 (512 contiguous bytes each) and 16
-// consecutive slots sit 16 bytes apart modulo 256 (no bank conflicts).
-constexpr uint32_t PF_RS = 2u * SF37_QK * 2u + 16u;  // 1040
-constexpr uint32_t PF_GRP = 16u * PF_RS;             // bytes of 32 slots
-constexpr uint32_t PF_ACT_BUF = PF_TB * PF_GRP;      // bytes of one LDS activation block
+constexpr uint32_t PF_NW = 4;           // waves per workgroup, 32 weight columns each
+constexpr uint32_t PF_GU_R = 16u * PF_NW;   // F rows per workgroup (16 gate + 16 up columns per wave)
+constexpr uint32_t PF_DN_R = 32u * PF_NW;   // output rows per workgroup
+// One (row, 256-block) of activations: 24 pieces of 16 bytes.  Group g, lane
+// half kh (codes 32 kh .. 32 kh + 31 of the group) has 12 dwords: the E3M2
+// fields of h (6 dwords), then the E2M3 fields of l; its piece j (0..2) is
+// c = 3 g + j, stored as piece 8 (c / 4) + 2 (c % 4) + kh.  In LDS, piece
+// 8 k + s of tile slot t is at k * PF_CHUNK + 128 t + 16 (s ^ (t % 8)): eight
+// lanes reading one piece of eight slots touch all banks, and a 64-lane
+// direct load fills eight slots' 128 contiguous bytes.
+constexpr uint32_t PF_BLK = 384;
+// ... and a record: the four groups' -gsum/64 as fp16 pairs, d, padding.
+constexpr uint32_t PF_REC = 32;
+constexpr uint32_t PF_CHUNK = PF_T * 128u;
+constexpr uint32_t PF_ACT_BUF = 3u * PF_CHUNK;
+static_assert(PF_BLK == SF37_QK * 12u / 8u && PF_BLK == 3u * 128u, "256 codes of 12 bits, three chunks");
 
 // Extents of the LDS direct loads.  A global_load_lds writes its 64 lanes'
 // bytes at M0 + 16 * lane (dwordx4) or M0 + 4 * lane (dword) whatever the
@@ -72,102 +74,130 @@ constexpr uint32_t PF_ACT_BUF = PF_TB * PF_GRP;      // bytes of one LDS activat
 // inside the buffer it targets.
 constexpr uint32_t DMA16_SPAN = 64u * 16u;
 constexpr uint32_t DMA4_SPAN = 64u * 4u;
-// pf_expert activation codes: M0 = buffer + gi * PF_GRP + t * PF_RS with slot
-// group gi <= PF_TB - 1 (8 waves: wave >> 2; 4 waves: k < 2) and t = 4 * wq +
-// (jj & 3) <= 15; lanes 32..63 fill slot t + 16, 512 bytes on.
-static_assert((PF_TB - 1u) * PF_GRP + 15u * PF_RS + DMA16_SPAN <= PF_ACT_BUF, "pf_expert code loads stay in their buffer");
-static_assert(DMA16_SPAN == 2u * 512u && 512u == 2u * SF37_QK, "one load = slots t and t + 16, 512 bytes each");
-static_assert(PF_RS >= 512u, "a slot row holds a block's 256 fp16 codes");
+// pf_expert codes: M0 = buffer + k * PF_CHUNK + r8 * 1024, chunk k <= 2, slot
+// octet r8 <= PF_T / 8 - 1
+static_assert(DMA16_SPAN == 8u * 128u && 2u * PF_CHUNK + (PF_T / 8u - 1u) * DMA16_SPAN + DMA16_SPAN <= PF_ACT_BUF,
+              "pf_expert code loads stay in their buffer");
+static_assert(PF_T / 8u == 2u * PF_NW, "each wave loads two slot octets (one per 32-pair block)");
+static_assert(PF_T * 16u == DMA16_SPAN && PF_T * 4u == DMA4_SPAN,
+              "pf_expert group-sum and scale loads fill exactly one buffer row each");
 
 // ---------------------------------------------------------------------------
-// Pair layouts.  Lane half kh of an MFMA holds 32 codes of every 64-group
-// (codes 32kh .. 32kh+31) as 16 pairs; pair P feeds MFMA P/4, dword P%4.
+// 6-bit fields.  A half-group's 32 fields are two 96-bit strings of 16: Q3,
+// the even codes (field i = code 2 i) and the odd ones (code 2 i + 1), so a
+// string is the lane's 96 payload bits (shifted by 3 for the odd codes) under
+// one mask; Q2, the codes of payload dword 0 and of dword 1, each dword
+// masked three ways: a 2-bit code keeps its bit in the dword, and codes 0, 3,
+// 6 .. 15 are fields of the string's first dword, 2, 5 .. 14 of the second,
+// 1, 4 .. 13 of the third.
 // ---------------------------------------------------------------------------
-// Q3 (3-bit codes at bit 3c of the lane's 96-bit string).  Window = the
-// string shifted right by the window offset; type = where the two codes sit
-// in the window: A1 bits 0 / 18, A2 bits 3 / 21, B1 bits 1 / 16, B2 bits 4 / 19.
-__constant__ uint8_t q3_lo_c[16] = {0, 1, 2, 3, 4, 5, 12, 13, 14, 15, 16, 22, 23, 24, 25, 26};
-__constant__ uint8_t q3_hi_c[16] = {6, 7, 8, 9, 10, 11, 17, 18, 19, 20, 21, 27, 28, 29, 30, 31};
-__constant__ uint8_t q3_ty_c[16] = {0, 1, 0, 1, 0, 1, 2, 3, 2, 3, 2, 2, 3, 2, 3, 2};
-// mantissa bit of the low / high code of each type (high relative to bit 16)
-__host__ __device__ constexpr uint32_t q3_plo(uint32_t ty) { return ty == 0 ? 0u : ty == 1 ? 3u : ty == 2 ? 1u : 4u; }
-__host__ __device__ constexpr uint32_t q3_phi(uint32_t ty) { return ty == 0 ? 2u : ty == 1 ? 5u : ty == 2 ? 0u : 3u; }
-__host__ __device__ constexpr uint32_t q3_mask(uint32_t ty) {
-    return (7u << q3_plo(ty)) | (7u << (16u + q3_phi(ty)));
+// mask of dword k of a string whose fields hold `bits`-bit codes
+__host__ __device__ constexpr uint32_t pf_mask(uint32_t k, uint32_t bits) {
+    uint32_t m = 0;
+    for (uint32_t i = 0; i < 32u; i++)
+        if ((32u * k + i) % 6u < bits) m |= 1u << i;
+    return m;
 }
-__host__ __device__ constexpr uint32_t pf_exp(uint32_t plo, uint32_t phi) {
-    return ((25u - plo) << 10) | ((25u - phi) << 26);
+static_assert((pf_mask(0, 2) | pf_mask(1, 2) | pf_mask(2, 2)) == 0xffffffffu &&
+                  (pf_mask(0, 2) & pf_mask(1, 2)) == 0 && (pf_mask(0, 2) & pf_mask(2, 2)) == 0,
+              "the three masks split a dword of 2-bit codes");
+
+// lanes exchanged within quads: xor 1 and xor 2
+template <int CTRL>
+__device__ __forceinline__ uint32_t dpp_quad(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, true);
 }
-__host__ __device__ constexpr uint32_t pf_mul(uint32_t plo, uint32_t phi) {
-    return (1u << plo) | (1u << (16u + phi));
-}
+constexpr int QUAD_XOR1 = 0xB1, QUAD_XOR2 = 0x4E;
 
 // ---------------------------------------------------------------------------
-// Activation kernel: Q8_K of one (row, 256-block) per wave, then the codes
-// in MFMA order as fp16, C per 64-group and d.
-// MFMA order of a block: position 64g + 32kh + 8m + e holds the code of
-// pair P = 4m + e/2 (low code if e even, high if odd) of lane half kh.
+// Activation kernel: Q8_K of one (row, 256-block) per wave, the codes as
+// 6-bit fields, -gsum/64 of the four groups and d.
 // ---------------------------------------------------------------------------
 template <bool Q3>
-__device__ __forceinline__ void pf_pos_code(uint32_t pos, uint32_t &code, int32_t &bias) {
-    const uint32_t kh = (pos >> 5) & 1u, m = (pos >> 3) & 3u, e = pos & 7u;
-    const uint32_t P = 4u * m + (e >> 1), half = e & 1u;
-    if (Q3) {
-        const uint32_t ty = q3_ty_c[P];
-        code = 32u * kh + (half ? q3_hi_c[P] : q3_lo_c[P]);
-        bias = (int32_t)(1u << (10u - (half ? q3_phi(ty) : q3_plo(ty)))) + 8;
-    } else {
-        const uint32_t k = P & 3u, qd = P >> 2;
-        code = 32u * kh + 16u * (qd >> 1) + 4u * (qd & 1u) + k + 8u * half;
-        bias = (int32_t)(1u << (10u - 2u * k)) + 4;
-    }
-}
-
-template <bool Q3>
-__global__ void __launch_bounds__(256) pf_act_kernel(_Float16 *__restrict__ codes, float *__restrict__ tab,
-                                                     const float *__restrict__ x, uint32_t nblk,
-                                                     uint32_t n_rows) {
+__global__ void __launch_bounds__(256) pf_act_kernel(uint32_t *__restrict__ codes, uint32_t *__restrict__ rec,
+                                                     const float *__restrict__ x, uint32_t nblk, uint32_t n_rows) {
     // each wave owns its LDS row and walks the (row, block) units wave by
     // wave over the grid; nothing is shared between waves
-    __shared__ int8_t qs[4][SF37_QK];
+    __shared__ __align__(16) uint8_t st[4][PF_BLK];
     const uint32_t wv = threadIdx.x >> 6, lane = threadIdx.x & 63u;
     const uint32_t units = nblk * n_rows, stride = gridDim.x * 4u;
-    // lane produces positions 4*lane .. 4*lane+3, all in group lane/16: their
-    // source codes and biases do not depend on the unit
-    const uint32_t g = lane >> 4;
-    uint32_t code[4];
-    int32_t bias[4];
-#pragma unroll
-    for (uint32_t c = 0; c < 4u; c++) pf_pos_code<Q3>(4u * (lane & 15u) + c, code[c], bias[c]);
+    uint8_t *row = st[wv];
+    // the lane's half-group (48 bytes), its quad in it, its place in the quad
+    const uint32_t hb = (lane >> 3) * 48u, quad = (lane >> 2) & 1u, qj = lane & 3u;
+    // piece `lane` (lanes < 24) of the output from the half-group order
+    const uint32_t pc = 4u * (lane >> 3) + ((lane & 7u) >> 1);
+    const uint32_t piece = (2u * (pc / 3u) + (lane & 1u)) * 48u + 16u * (pc % 3u);
     for (uint32_t u = blockIdx.x * 4u + wv; u < units; u += stride) {
-        const float *xb = x + (uint64_t)u * SF37_QK + 4u * lane;
-        float v[4];
-#pragma unroll
-        for (int k = 0; k < 4; k++) v[k] = xb[k];
+        const float4 xv = *(const float4 *)(x + (uint64_t)u * SF37_QK + 4u * lane);
+        const float v[4] = {xv.x, xv.y, xv.z, xv.w};
         int8_t q[4];
-        int gs;
-        const float d = q8k_codes4(v, q, gs);
-        (void)gs;
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the previous unit's reads are done
+        int gsum;
+        const float d = q8k_codes4(v, q, gsum);
+        // magnitudes and signs, a byte per code; h = magnitude / 16, l the rest
+        uint32_t m = 0, sg = 0;
 #pragma unroll
-        for (int k = 0; k < 4; k++) qs[wv][4u * lane + k] = q[k];
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // this unit's codes are in LDS
-        __builtin_amdgcn_wave_barrier();
-        int32_t s = 0;
-        _Float16 h[4];
-#pragma unroll
-        for (uint32_t c = 0; c < 4u; c++) {
-            const int32_t a = qs[wv][64u * g + code[c]];
-            h[c] = (_Float16)a;
-            s += bias[c] * a;
+        for (int k = 0; k < 4; k++) {
+            const int a = q[k];
+            m |= (uint32_t)(a < 0 ? -a : a) << (8 * k);
+            sg |= (a < 0 ? 0x20u : 0u) << (8 * k);
         }
-        s = wave_sum_i32_width(s, 16);
-        typedef _Float16 h4 __attribute__((ext_vector_type(4)));
-        const h4 hv = {h[0], h[1], h[2], h[3]};
-        *(h4 *)(codes + (uint64_t)u * SF37_QK + 4u * lane) = hv;
-        float *tb = tab + (uint64_t)u * PF_TAB;
-        if ((lane & 15u) == 0u) tb[g] = (float)(-s);
-        if (lane == 0u) tb[4] = d;
+        const uint32_t hm = (m >> 4) & 0x0f0f0f0fu, h8 = hm & 0x08080808u;
+        // E3M2 of 2 h: 0, 16, 20, 22, 24, 25, 26, 27 by table, 28 for h = 8
+        // (for which the byte select reads the sign of 0x10: zero)
+        uint32_t eh = vperm(0x1B1A1918u, 0x16141000u, hm);
+        eh |= (h8 >> 1) | h8 | (h8 << 1) | sg;
+        const uint32_t el = (m & 0x0f0f0f0fu) | sg;
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the previous unit's reads are done
+        if constexpr (Q3) {
+#pragma unroll
+            for (uint32_t k = 0; k < 4u; k++) {   // even h, odd h, even l, odd l
+                const uint32_t e = k < 2u ? eh : el;
+                const uint32_t two = (k & 1u) ? ((e >> 8) & 0x3fu) | ((e >> 18) & 0xfc0u)
+                                              : (e & 0x3fu) | ((e >> 10) & 0xfc0u);
+                uint32_t w = two << (12u * (lane & 1u));
+                w |= dpp_quad<QUAD_XOR1>(w);                       // 24 bits of the lane pair
+                const uint32_t t = dpp_quad<QUAD_XOR2>(w);         // the other pair's
+                if (qj == 0u) {                                    // 48 bits of the quad
+                    uint16_t *o = (uint16_t *)(row + hb + 12u * k + 6u * quad);
+                    const uint32_t lo = w | (t << 24);
+                    o[0] = (uint16_t)lo;
+                    o[1] = (uint16_t)(lo >> 16);
+                    o[2] = (uint16_t)(t >> 8);
+                }
+            }
+        } else {
+#pragma unroll
+            for (uint32_t k = 0; k < 2u; k++) {   // h, l
+                const uint32_t e = k ? el : eh;
+                // the lane's codes 4 qj .. 4 qj + 3 by the dword of the string
+                // they go to: X0 has codes 0 and 3, X1 code 1, X2 code 2
+                const uint32_t x0 = (e & 0x3fu) | ((e >> 18) & 0xfc0u), x1 = ((e >> 8) & 0x3fu) << 2,
+                               x2 = ((e >> 16) & 0x3fu) << 4;
+                const uint32_t r0 = qj == 1u ? x2 : qj == 2u ? x1 : x0;
+                const uint32_t r1 = qj == 1u ? x1 : qj == 2u ? x0 : x2;
+                const uint32_t r2 = qj == 1u ? x0 : qj == 2u ? x2 : x1;
+                uint32_t d0 = r0 << (8u * qj), d1 = r1 << (8u * qj), d2 = r2 << (8u * qj);
+                // fields of codes 15 and 14 that run into the next dword
+                d1 |= qj == 3u ? x0 >> 8 : 0u;
+                d2 |= qj == 3u ? x2 >> 8 : 0u;
+                d0 |= dpp_quad<QUAD_XOR1>(d0);
+                d1 |= dpp_quad<QUAD_XOR1>(d1);
+                d2 |= dpp_quad<QUAD_XOR1>(d2);
+                d0 |= dpp_quad<QUAD_XOR2>(d0);
+                d1 |= dpp_quad<QUAD_XOR2>(d1);
+                d2 |= dpp_quad<QUAD_XOR2>(d2);
+                if (qj < 3u) *(uint32_t *)(row + hb + 24u * k + 12u * quad + 4u * qj) = qj == 0u ? d0 : qj == 1u ? d1 : d2;
+            }
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // this unit's fields are in LDS
+        __builtin_amdgcn_wave_barrier();
+        if (lane < 24u) *(uint4 *)((uint8_t *)codes + (uint64_t)u * PF_BLK + 16u * lane) = *(const uint4 *)(row + piece);
+        if ((lane & 15u) == 0u) {
+            const _Float16 hi = (_Float16)((float)(gsum >> 4) * -0.25f), lo = (_Float16)((float)(gsum & 15) * -0.015625f);
+            rec[(uint64_t)u * (PF_REC / 4u) + (lane >> 4)] = (uint32_t)__builtin_bit_cast(unsigned short, hi) |
+                                                             (uint32_t)__builtin_bit_cast(unsigned short, lo) << 16;
+        }
+        if (lane == 0u) rec[(uint64_t)u * (PF_REC / 4u) + 4u] = __builtin_bit_cast(uint32_t, d);
     }
 }
 
@@ -218,26 +248,6 @@ __global__ void __launch_bounds__(1024) pf_tiles_kernel(uint32_t *__restrict__ t
 }
 
 // ---------------------------------------------------------------------------
-// Tables in dispatch order: tabs[(b * 5 + a) * stride + s] = tab[row(s)][b][a]
-// for sorted position s (row = pair / div: the token for x, the pair for the
-// mid), a = C0..C3, d.  A tile's entries are then contiguous.
-// ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(256) pf_tab_sort_kernel(float *__restrict__ tabs, const float *__restrict__ tab,
-                                                          const uint32_t *__restrict__ sorted, uint32_t n_pairs,
-                                                          uint32_t nblk, uint32_t div, uint32_t stride) {
-    const uint32_t s = blockIdx.x * 256u + threadIdx.x, b = blockIdx.y;
-    if (s >= n_pairs) return;
-    const float *t = tab + ((uint64_t)(sorted[s] / div) * nblk + b) * PF_TAB;
-    const float4 c = *(const float4 *)t;
-    float *o = tabs + (uint64_t)b * 5u * stride + s;
-    o[0] = c.x;
-    o[(uint64_t)stride] = c.y;
-    o[2ull * stride] = c.z;
-    o[3ull * stride] = c.w;
-    o[4ull * stride] = t[4];
-}
-
-// ---------------------------------------------------------------------------
 // LDS direct loads (global -> LDS, no registers).  Issued through inline asm
 // so the compiler does not wait for them before unrelated LDS reads; the
 // kernel waits with s_waitcnt vmcnt(0) + barrier before reading the buffer.
@@ -266,89 +276,95 @@ __device__ __forceinline__ void lds_dma4(uint32_t lds, uint32_t voff, const void
                  : "memory");
 }
 __device__ __forceinline__ void wait_vm0() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
-// All but the newest PF_DMA_PER_BLOCK vector-memory operations of the wave
-// done: the activation loads issued for the block after next stay in flight
-// (8-wave workgroups, three buffers).
-constexpr int PF_DMA_PER_BLOCK = 5;   // 4 code rows + 1 table row per wave and block
-static_assert(PF_DMA_PER_BLOCK == 5, "the count in wait_vm_keep_next");
-__device__ __forceinline__ void wait_vm_keep_next() { asm volatile("s_waitcnt vmcnt(5)" ::: "memory"); }
-
-// After wait_vm0, mark a block's weight words as just defined: the compiler
-// then knows no load is pending on them and does not place its own
-// s_waitcnt vmcnt inside the compute (which would also wait for the next
-// block's LDS direct loads, issued earlier in program order).
-struct q3_raw;
-struct q2_raw;
 
 __device__ __forceinline__ uint32_t lds_addr(const void *p) { return (uint32_t)(uintptr_t)p; }
+
+// Direct loads of a block's records, a slot per lane: wave 0 the group sums,
+// wave 1 the scales.  One asm statement with the branches inside, so that the
+// code around it stays one block for the compiler (which otherwise moves the
+// fmas before a branch behind it).
+__device__ __forceinline__ void pf_rec_load(uint32_t wave, uint32_t gs_lds, uint32_t d_lds, uint32_t voff,
+                                            const uint8_t *rec) {
+    asm volatile("s_cmp_lg_u32 %0, 0\n\t"
+                 "s_cbranch_scc1 .Lpfg%=\n\t"
+                 "s_mov_b32 m0, %1\n\t"
+                 "s_nop 0\n\t"
+                 "global_load_lds_dwordx4 %3, %4\n"
+                 ".Lpfg%=:\n\t"
+                 "s_cmp_lg_u32 %0, 1\n\t"
+                 "s_cbranch_scc1 .Lpfd%=\n\t"
+                 "s_mov_b32 m0, %2\n\t"
+                 "s_nop 0\n\t"
+                 "global_load_lds_dword %3, %5\n"
+                 ".Lpfd%=:" ::"s"(__builtin_amdgcn_readfirstlane(wave)),
+                 "s"(__builtin_amdgcn_readfirstlane(gs_lds)), "s"(__builtin_amdgcn_readfirstlane(d_lds)), "v"(voff),
+                 "s"(sgpr_ptr(rec)), "s"(sgpr_ptr(rec + 16))
+                 : "memory", "scc");
+}
 
 struct pf_params {
     float *mid, *gate_out, *up_out, *down_pair;
     const uint8_t *w0, *w1;        // gate / up (Q3) or down (Q2)
-    const _Float16 *act;           // [rows][nblk * 256] codes in MFMA order
-    const float *tab;              // [nblk][5][tab_stride] tables in dispatch order
+    const uint8_t *act;            // [rows][nblk][PF_BLK] fields
+    const uint8_t *rec;            // [rows][nblk][PF_REC]
     const uint32_t *tiles;
     const uint32_t *sorted;
     const float *weights;
-    uint32_t topk, nblk, out_rows, n_rt, tab_stride;
+    uint32_t topk, nblk, out_rows, n_rt;
     float clamp;
 };
 
-// Weight bytes of one lane for one block.
-struct q3_raw {
-    uint32_t h[4];      // header dwords (scales, zero points)
-    uint32_t w[4][4];   // per group: 16 aligned bytes holding the lane's 12
+// Weight bytes of one lane for one Q3 block: the header dwords (scales, zero
+// points) and per group the aligned dwords that hold the half's 12 bytes:
+// three of each when the block starts on a dword, four in an odd block, which
+// starts two bytes in.
+// (Vector types, so that the loop carries each load's result as the register
+// tuple it was loaded into: as single words they are copied at the end of an
+// iteration, which waits for them there.)
+typedef uint32_t u32x4a __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t u32x3a __attribute__((ext_vector_type(3), aligned(4)));
+template <bool ODD> struct q3_raw {
+    typedef typename std::conditional<ODD, u32x4a, u32x3a>::type vec;
+    vec h, w[4];
 };
+
+// hp: the header's first dword (odd blocks: two bytes before the block); pp:
+// the dword at which group 0's payload starts
+template <bool ODD>
+__device__ __forceinline__ void q3_load(q3_raw<ODD> &r, const uint8_t *hp, const uint8_t *pp) {
+    typedef typename q3_raw<ODD>::vec vec;
+    r.h = *(const vec *)hp;
+#pragma unroll
+    for (int g = 0; g < 4; g++) r.w[g] = *(const vec *)(pp + 24 * g);
+}
+
+// After a wait for them, mark a block's weight words as just defined: the
+// compiler then knows no load is pending on them and places no s_waitcnt
+// vmcnt of its own inside the compute (which would also wait for the loads
+// and LDS direct loads issued since).
+template <bool ODD>
+__device__ __forceinline__ void raw_ready(q3_raw<ODD> &r) {
+    asm volatile("" : "+v"(r.h), "+v"(r.w[0]), "+v"(r.w[1]), "+v"(r.w[2]), "+v"(r.w[3]));
+}
+
 struct q2_raw {
     uint32_t h[3];
     uint32_t w[4][2];
 };
-
-
-__device__ __forceinline__ void raw_ready(q3_raw &r) {
-    asm volatile("" : "+v"(r.h[0]), "+v"(r.h[1]), "+v"(r.h[2]), "+v"(r.h[3]), "+v"(r.w[0][0]), "+v"(r.w[0][1]),
-                 "+v"(r.w[0][2]), "+v"(r.w[0][3]), "+v"(r.w[1][0]), "+v"(r.w[1][1]), "+v"(r.w[1][2]),
-                 "+v"(r.w[1][3]), "+v"(r.w[2][0]), "+v"(r.w[2][1]), "+v"(r.w[2][2]), "+v"(r.w[2][3]),
-                 "+v"(r.w[3][0]), "+v"(r.w[3][1]), "+v"(r.w[3][2]), "+v"(r.w[3][3]));
-}
-
-typedef uint32_t u32x4a __attribute__((ext_vector_type(4), aligned(4)));
-typedef uint32_t u32x3a __attribute__((ext_vector_type(3), aligned(4)));
-typedef uint32_t u32x2a __attribute__((ext_vector_type(2), aligned(4)));
-
-// Q3 words as dword loads (no register tuples): the words go straight into
-// the registers the loop carries them in, so no copy waits for the data.
-// (Contiguous half-block loads with lane swaps, as the Q2 blocks below,
-// measured 1.5 % slower here: twelve swaps per block cost more VALU than
-// the sixteen fewer loads save in this VALU-bound kernel.)
-__device__ __forceinline__ void q3_load(q3_raw &r, const uint8_t *hp, const uint8_t *pp) {
-    const uint32_t *h = (const uint32_t *)hp;
-#pragma unroll
-    for (int i = 0; i < 4; i++) r.h[i] = h[i];
-#pragma unroll
-    for (int g = 0; g < 4; g++) {
-        const uint32_t *q = (const uint32_t *)(pp + 24 * g);
-#pragma unroll
-        for (int i = 0; i < 4; i++) r.w[g][i] = q[i];
-    }
-}
-
-
 // What a lane loads of a Q2 block (21 dwords): dwords 8 kh .. 8 kh + 10,
 // contiguous (three loads instead of eleven); pf_words then trades what each
 // half needs from the other with v_permlane32_swap (lanes l and l + 32 hold
 // the same row).
 struct q2_half {
-    uint32_t w[11];
+    u32x4a a, b;
+    u32x3a c;
 };
-__device__ __forceinline__ void raw_ready(q2_half &r) {
-    asm volatile("" : "+v"(r.w[0]), "+v"(r.w[1]), "+v"(r.w[2]), "+v"(r.w[3]), "+v"(r.w[4]), "+v"(r.w[5]),
-                 "+v"(r.w[6]), "+v"(r.w[7]), "+v"(r.w[8]), "+v"(r.w[9]), "+v"(r.w[10]));
-}
+__device__ __forceinline__ void raw_ready(q2_half &r) { asm volatile("" : "+v"(r.a), "+v"(r.b), "+v"(r.c)); }
 __device__ __forceinline__ void q2_load_half(q2_half &r, const uint8_t *bp, uint32_t kh) {
     const uint32_t *q = (const uint32_t *)bp + 8u * kh;
-#pragma unroll
-    for (int i = 0; i < 11; i++) r.w[i] = q[i];
+    r.a = *(const u32x4a *)q;
+    r.b = *(const u32x4a *)(q + 4);
+    r.c = *(const u32x3a *)(q + 8);
 }
 // q2_raw of both halves: the header dwords 0..2 and group g's dwords
 // 3 + 4 g + 2 kh, +1.  permlane32_swap(A, B) gives [A of lanes 0-31, B of
@@ -357,33 +373,24 @@ __device__ __forceinline__ void q2_load_half(q2_half &r, const uint8_t *bp, uint
 // for both halves, the second the same word of group 2 or 3 (8 dwords on);
 // a swap of dword j with itself hands both halves header dword j.
 __device__ __forceinline__ q2_raw pf_words(const q2_half &h) {
+    const uint32_t w[11] = {h.a[0], h.a[1], h.a[2], h.a[3], h.b[0], h.b[1], h.b[2], h.b[3], h.c[0], h.c[1], h.c[2]};
     q2_raw r;
 #pragma unroll
-    for (int j = 0; j < 3; j++) r.h[j] = __builtin_amdgcn_permlane32_swap(h.w[j], h.w[j], false, false)[0];
+    for (int j = 0; j < 3; j++) r.h[j] = __builtin_amdgcn_permlane32_swap(w[j], w[j], false, false)[0];
 #pragma unroll
     for (int g = 0; g < 2; g++) {
 #pragma unroll
         for (int i = 0; i < 2; i++) {
-            const auto v = __builtin_amdgcn_permlane32_swap(h.w[3 + 4 * g + i], h.w[5 + 4 * g + i], false, false);
+            const auto v = __builtin_amdgcn_permlane32_swap(w[3 + 4 * g + i], w[5 + 4 * g + i], false, false);
             r.w[g][i] = v[0];
             r.w[g + 2][i] = v[1];
         }
     }
     return r;
 }
-__device__ __forceinline__ const q3_raw &pf_words(const q3_raw &r) { return r; }
-
-// 32 bits of the lane's string starting at bit SH + o of the loaded words.
-template <int SH, int O>
-__device__ __forceinline__ uint32_t q3_win(const uint32_t *w) {
-    constexpr int a = SH + O, k = a >> 5, s = a & 31;
-    if constexpr (s == 0) return w[k];
-    else return align_bits(w[k + 1], w[k], (uint32_t)s);
-}
-
 // f16 scale of group g, zero point of group g from the header bits at SH.
-template <int SH>
-__device__ __forceinline__ float hdr_scale(const uint32_t *h, int g) {
+template <int SH, typename H>
+__device__ __forceinline__ float hdr_scale(const H &h, int g) {
     const int a = SH + 16 * g;
     return sf37_f16(h[a >> 5] >> (a & 31));
 }
@@ -393,207 +400,141 @@ __device__ __forceinline__ uint32_t hdr_zp(const uint32_t *h, int g) {
     return (h[a >> 5] >> (a & 31)) & 0xffu;
 }
 
-// Q3 / Q2 dequantisation of part (0: pair words 0..7, 1: words 8..15) of group g.
-template <bool Q3, int SH, int PART, typename RAW>
-__device__ __forceinline__ void pf_dequant(const RAW &r, int g, uint32_t out[16]) {
+// A block's weight words into r.
+template <bool Q3, bool ODD> using pf_raw_t = typename std::conditional<Q3, q3_raw<ODD>, q2_half>::type;
+template <bool Q3, bool ODD>
+__device__ __forceinline__ void pf_wload(pf_raw_t<Q3, ODD> &r, const uint8_t *wrow, uint32_t bn, uint32_t kh) {
     if constexpr (Q3) {
-        const uint32_t k = 8u - (hdr_zp<SH>(r.h, g) & 7u);
-        const uint32_t *w = r.w[g];
-        constexpr uint32_t mA1 = q3_mask(0), mA2 = q3_mask(1), mB1 = q3_mask(2), mB2 = q3_mask(3);
-        const uint32_t cB1 = pf_exp(1, 0) + k * pf_mul(1, 0), cB2 = pf_exp(4, 3) + k * pf_mul(4, 3);
-        uint32_t x;
-        if constexpr (PART == 0) {
-            const uint32_t cA1 = pf_exp(0, 2) + k * pf_mul(0, 2), cA2 = pf_exp(3, 5) + k * pf_mul(3, 5);
-            x = q3_win<SH, 0>(w);  out[0] = (x & mA1) + cA1;  out[1] = (x & mA2) + cA2;
-            x = q3_win<SH, 6>(w);  out[2] = (x & mA1) + cA1;  out[3] = (x & mA2) + cA2;
-            x = q3_win<SH, 12>(w); out[4] = (x & mA1) + cA1;  out[5] = (x & mA2) + cA2;
-            x = q3_win<SH, 35>(w); out[6] = (x & mB1) + cB1;  out[7] = (x & mB2) + cB2;
-        } else {
-            x = q3_win<SH, 41>(w); out[8] = (x & mB1) + cB1;  out[9] = (x & mB2) + cB2;
-            x = q3_win<SH, 47>(w); out[10] = (x & mB1) + cB1;
-            x = q3_win<SH, 65>(w); out[11] = (x & mB1) + cB1; out[12] = (x & mB2) + cB2;
-            x = q3_win<SH, 71>(w); out[13] = (x & mB1) + cB1; out[14] = (x & mB2) + cB2;
-            x = q3_win<SH, 77>(w); out[15] = (x & mB1) + cB1;
-        }
-    } else {
-        const uint32_t k = 4u - (hdr_zp<0>(r.h, g) & 3u);
-        const uint32_t u = r.w[g][PART];
-#pragma unroll
-        for (uint32_t h = 0; h < 2u; h++) {
-            const uint32_t x = h ? (u >> 8) : u;
-#pragma unroll
-            for (uint32_t j = 0; j < 4u; j++)
-                out[8 * PART + 4u * h + j] =
-                    (x & (0x00030003u << (2u * j))) + pf_exp(2u * j, 2u * j) + k * pf_mul(2u * j, 2u * j);
-        }
-    }
-}
-
-// One 256-block of the tile.  Chains c = (group g, token block i), 4*NTB of
-// them, each = 4 MFMAs on accumulator D = C(g, i).  Stage c calls pre(c)
-// (a slice of the next block's global loads, so a stalled memory issue
-// overlaps MFMAs already in flight), issues the LDS loads of chain c+1,
-// part of the next group's dequantisation, the MFMAs of chain c and the
-// epilogue blk = fma(s_g, D, blk) of chain c-1; stages are fenced so the
-// compiler interleaves within a stage only.  Then acc = fma(d, blk, acc)
-// per token block.
-template <bool Q3, int SH, int NTB, typename RAW, typename PRE>
-__device__ __forceinline__ void pf_block(const RAW &r, const uint8_t *act_lds, const float *cd_lds,
-                                         uint32_t kh, uint32_t col, float (*acc)[16], f16v blk[PF_TB],
-                                         PRE &&pre) {
-    constexpr int NC = 4 * NTB;
-    const uint8_t *a_lane = act_lds + (col & 15u) * PF_RS + (col >> 4) * 512u + 64u * kh;
-    const float *c_lane = cd_lds + 4u * kh;
-    uint32_t bw[2][16];
-    float s[4];
-#pragma unroll
-    for (int g = 0; g < 4; g++) s[g] = hdr_scale<Q3 ? SH : 0>(r.h, g);
-    pf_dequant<Q3, SH, 0>(r, 0, bw[0]);
-    pf_dequant<Q3, SH, 1>(r, 0, bw[0]);
-    f16v D[3];
-    h8 A[2][4];
-    auto load = [&](int c, f16v &d, h8 *a) {
-        const int g = c / NTB, i = c % NTB;
-#pragma unroll
-        for (int jj = 0; jj < 4; jj++) {
-            const float4 v = *(const float4 *)(c_lane + g * PF_T + 32 * i + 8 * jj);
-            d[4 * jj] = v.x; d[4 * jj + 1] = v.y; d[4 * jj + 2] = v.z; d[4 * jj + 3] = v.w;
-        }
-#pragma unroll
-        for (int m = 0; m < 4; m++) a[m] = *(const h8 *)(a_lane + i * PF_GRP + (8 * g + m) * 16);
-    };
-    load(0, D[0], A[0]);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int c = 0; c < NC; c++) {
-        const int g = c / NTB, i = c % NTB;
-        pre(c, NC);
-        if (c + 1 < NC) load(c + 1, D[(c + 1) % 3], A[(c + 1) & 1]);
-        if (g < 3) {
-            constexpr int P0 = NTB >= 3 ? 1 : 0, P1 = NTB >= 3 ? 2 : NTB - 1;
-            if (i == P0) pf_dequant<Q3, SH, 0>(r, g + 1, bw[(g + 1) & 1]);
-            if (i == P1) pf_dequant<Q3, SH, 1>(r, g + 1, bw[(g + 1) & 1]);
-        }
-        {
-            const uint32_t *bb = bw[g & 1];
-#pragma unroll
-            for (int m = 0; m < 4; m++) {
-                typedef uint32_t u4 __attribute__((ext_vector_type(4)));
-                const u4 t = {bb[4 * m], bb[4 * m + 1], bb[4 * m + 2], bb[4 * m + 3]};
-                D[c % 3] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[c & 1][m], __builtin_bit_cast(h8, t), D[c % 3], 0, 0, 0);
-            }
-        }
-        if (c > 0) {
-            const int gp = (c - 1) / NTB, ip = (c - 1) % NTB;
-#pragma unroll
-            for (int r2 = 0; r2 < 16; r2++)
-                blk[ip][r2] = __builtin_fmaf(s[gp], D[(c - 1) % 3][r2], gp == 0 ? 0.0f : blk[ip][r2]);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-    }
-#pragma unroll
-    for (int r2 = 0; r2 < 16; r2++)
-        blk[NTB - 1][r2] = __builtin_fmaf(s[3], D[(NC - 1) % 3][r2], blk[NTB - 1][r2]);
-#pragma unroll
-    for (int i = 0; i < NTB; i++) {
-#pragma unroll
-        for (int jj = 0; jj < 4; jj++) {
-            const float4 d = *(const float4 *)(c_lane + 4 * PF_T + 32 * i + 8 * jj);
-            acc[i][4 * jj] = __builtin_fmaf(d.x, blk[i][4 * jj], acc[i][4 * jj]);
-            acc[i][4 * jj + 1] = __builtin_fmaf(d.y, blk[i][4 * jj + 1], acc[i][4 * jj + 1]);
-            acc[i][4 * jj + 2] = __builtin_fmaf(d.z, blk[i][4 * jj + 2], acc[i][4 * jj + 2]);
-            acc[i][4 * jj + 3] = __builtin_fmaf(d.w, blk[i][4 * jj + 3], acc[i][4 * jj + 3]);
-        }
-    }
-}
-
-template <bool Q3> using pf_raw_t = typename std::conditional<Q3, q3_raw, q2_half>::type;
-
-// One tile's view for the routed kernels: its expert, pairs and weight row,
-// and the per-lane direct-load offsets of its activation rows.
-template <bool Q3>
-struct pf_item {
-    uint32_t e, p0, cnt, ntb;
-    const uint8_t *wrow;
-    uint32_t wcol;
-    uint32_t voff[pf_cfg<Q3>::NW == 8u ? 4 : 1];
-    uint32_t rowoff_c[pf_cfg<Q3>::NW == 8u ? 1 : 2];
-};
-
-// A block's weight words into r (even blocks start dword-aligned, odd Q3
-// blocks 2 bytes in).
-template <bool Q3>
-__device__ __forceinline__ void pf_wload(pf_raw_t<Q3> &r, const uint8_t *wrow, uint32_t bn, uint32_t kh) {
-    if constexpr (Q3) {
-        const uint32_t o = SF37_Q3_BYTES * bn;
-        q3_load(r, wrow + (o & ~3u), wrow + ((o + 12u + 12u * kh) & ~3u));
+        const uint8_t *hp = wrow + (uint64_t)SF37_Q3_BYTES * bn - (ODD ? 2 : 0);
+        q3_load<ODD>(r, hp, hp + 12u + 12u * kh);
     } else {
         q2_load_half(r, wrow + (uint64_t)SF37_Q2_BYTES * bn, kh);
     }
 }
 
-// The block loop for NTB 32-pair blocks (the tile's pair count rounded up).
-// On entry block 0's weights are loading into ra and its activation rows
-// (with NBUF = 3, block 1's too) are issued; on exit every load is done.
-//
-// Pipeline: a block's weight words (registers) are loaded one block
-// ahead.  Three activation buffers (8 waves): the activation rows and
-// tables of block b+2 are loaded during block b, spread over its stages,
-// and the top of block b+1 waits for all but those newest
-// PF_DMA_PER_BLOCK loads.  Two buffers (4 waves): those of block b+1 are
-// issued at the start of block b, and the top of block b+1 waits for
-// every load.  Past the last block the loads repeat block nblk-1 (its
-// buffer then receives the same bytes again; uniform code, no branch
-// inside the stages); the final wait keeps no load in flight at the end
-// of the workgroup.
-template <bool Q3, int NTB, typename ISSUE>
-__device__ __forceinline__ void pf_loop(const pf_params &p, const uint8_t *wrow, ISSUE &&issue_act,
-                                        uint8_t (*s_act)[PF_ACT_BUF], float (*s_cd)[PF_CD_ROWS * PF_T],
-                                        uint32_t kh, uint32_t col, pf_raw_t<Q3> &ra, float (*acc)[16]) {
-    const uint32_t nblk = p.nblk;
-    f16v blk[PF_TB];
+// All of the wave's vector-memory operations done but the newest block of
+// weight words (the loads pf_wload makes: five, or three for Q2).
+template <bool Q3>
+__device__ __forceinline__ void wait_vm_keep_weights() {
+    if constexpr (Q3) asm volatile("s_waitcnt vmcnt(5)" ::: "memory");
+    else asm volatile("s_waitcnt vmcnt(3)" ::: "memory");
+}
+
+// A block's weights as MFMA operands: 4 groups x 32 columns x 64 codes.
+struct pf_b {
+    uint32_t w[4][6];   // E2M3 fields, code / 8
+    uint32_t z[4];      // zp as an fp16 pair (lane half 0; zero in half 1)
+    float s[4];         // 64 x the group's scale
+};
+
+// zt: fp16 high bytes of 0..7 for the zero points (zero in lane half 1, whose
+// share of the fp16 MFMA's K is unused)
+template <bool Q3, int SH, typename RAW>
+__device__ __forceinline__ void pf_dequant(pf_b &o, const RAW &r, const uint32_t zt[2]) {
 #pragma unroll
-    for (int i = 0; i < NTB; i++)
+    for (int g = 0; g < 4; g++) {
+        const auto w = r.w[g];
+        if constexpr (Q3) {
+            constexpr uint32_t m0 = pf_mask(0, 3), m1 = pf_mask(1, 3), m2 = pf_mask(2, 3);
+            if constexpr (SH == 0) {
+                o.w[g][0] = w[0] & m0;
+                o.w[g][1] = w[1] & m1;
+                o.w[g][2] = w[2] & m2;
+                o.w[g][5] = (w[2] >> 3) & m2;
+            } else {
+                o.w[g][0] = align_bits(w[1], w[0], SH) & m0;
+                o.w[g][1] = align_bits(w[2], w[1], SH) & m1;
+                o.w[g][2] = align_bits(w[3], w[2], SH) & m2;
+                o.w[g][5] = align_bits(w[3], w[2], SH + 3) & m2;
+            }
+            o.w[g][3] = align_bits(w[1], w[0], SH + 3) & m0;
+            o.w[g][4] = align_bits(w[2], w[1], SH + 3) & m1;
+        } else {
 #pragma unroll
-        for (int r2 = 0; r2 < 16; r2++) acc[i][r2] = 0.0f;
-    constexpr uint32_t NBUF = pf_cfg<Q3>::NBUF;
-    const uint32_t last = nblk - 1u;
-    auto clampb = [&](uint32_t x) { return x < nblk ? x : last; };
-    auto top = [&]() {
-        if constexpr (NBUF == 3u) wait_vm_keep_next();
-        else wait_vm0();
-    };
-    pf_raw_t<Q3> rb;
-    // the block's loads: weights of bn into r, activations of ba
-    auto pre = [&](pf_raw_t<Q3> &r, uint32_t bn, uint32_t ba, int c, int nc) {
-        if (c == 0) pf_wload<Q3>(r, wrow, bn, kh);
-        if constexpr (NBUF == 3u) issue_act(ba, c, nc);
-        else if (c == 0) issue_act(ba, 0, 1);
-    };
-    constexpr int SH2 = Q3 ? 16 : 0;   // bit offset of an odd block's string in its words
-    for (uint32_t b = 0; b < nblk; b += 2u) {
-        top();
-        raw_ready(ra);
-        __syncthreads();
-        const uint32_t b1 = clampb(b + 1u), b2 = clampb(b + 2u), b3 = clampb(b + 3u);
-        pf_block<Q3, 0, NTB>(pf_words(ra), s_act[b % NBUF], s_cd[b % NBUF], kh, col, acc, blk,
-                             [&](int c, int nc) { pre(rb, b1, NBUF == 3u ? b2 : b1, c, nc); });
-        if (b + 1u < nblk) {
-            top();
-            raw_ready(rb);
-            __syncthreads();
-            pf_block<Q3, SH2, NTB>(pf_words(rb), s_act[(b + 1u) % NBUF], s_cd[(b + 1u) % NBUF], kh, col, acc, blk,
-                                   [&](int c, int nc) { pre(ra, b2, NBUF == 3u ? b3 : b2, c, nc); });
+            for (int j = 0; j < 2; j++)
+#pragma unroll
+                for (uint32_t k = 0; k < 3u; k++) o.w[g][3 * j + k] = w[j] & pf_mask(k, 2);
         }
     }
-    wait_vm0();
+    const uint32_t zps = (SH ? align_bits(r.h[SH ? 3 : 2], r.h[2], SH) : r.h[2]) & (Q3 ? 0x07070707u : 0x03030303u);
+    const uint32_t zh = vperm(zt[1], zt[0], zps);
+#pragma unroll
+    for (uint32_t g = 0; g < 4u; g++) {
+        o.z[g] = vperm(zh, zh, g << 8 | g << 24 | 0x000c000cu);
+        o.s[g] = 64.0f * hdr_scale<SH>(r.h, (int)g);
+    }
+}
+
+typedef int v8i __attribute__((ext_vector_type(8)));
+constexpr int FMT_E2M3 = 2, FMT_E3M2 = 3;
+// D += A (format FA) x B (E2M3) over one 64-group; only the first six dwords
+// of each operand are read, and zero scale operands select the unscaled form
+template <int FA>
+__device__ __forceinline__ f16v pf_mfma6(const uint32_t *a, const uint32_t *b, f16v c) {
+    const v8i A = {(int)a[0], (int)a[1], (int)a[2], (int)a[3], (int)a[4], (int)a[5], 0, 0};
+    const v8i B = {(int)b[0], (int)b[1], (int)b[2], (int)b[3], (int)b[4], (int)b[5], 0, 0};
+    return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(A, B, c, FA, FMT_E2M3, 0, 0, 0, 0);
+}
+
+// One 256-block of the tile.  Chain c = (pair block i, group g): three MFMAs
+// from zero; stage c issues its LDS reads and MFMAs and the epilogue
+// blk = fma(s_g, D, blk) of chain c - 1; stages are fenced so the compiler
+// interleaves within a stage only.  After a pair block's group 3,
+// acc = fma(d, blk, acc).
+template <int NTB>
+__device__ __forceinline__ void pf_block(const pf_b &b, const uint8_t *act_lds, const uint8_t *gs_lds,
+                                         const float *d_lds, const uint32_t aofs[4], uint32_t kh, uint32_t col,
+                                         f16v *acc) {
+    constexpr int NC = 4 * NTB;
+    f16v D[2], blk;
+    uint4 G;
+    auto finish = [&](int c) {
+        const int i = c >> 2, g = c & 3;
+#pragma unroll
+        for (int r = 0; r < 16; r++) blk[r] = __builtin_fmaf(b.s[g], D[c & 1][r], g == 0 ? 0.0f : blk[r]);
+        if (g == 3) {
+#pragma unroll
+            for (int jj = 0; jj < 4; jj++) {
+                const float4 d = *(const float4 *)(d_lds + 32 * i + 8 * jj + 4u * kh);
+                acc[i][4 * jj] = __builtin_fmaf(d.x, blk[4 * jj], acc[i][4 * jj]);
+                acc[i][4 * jj + 1] = __builtin_fmaf(d.y, blk[4 * jj + 1], acc[i][4 * jj + 1]);
+                acc[i][4 * jj + 2] = __builtin_fmaf(d.z, blk[4 * jj + 2], acc[i][4 * jj + 2]);
+                acc[i][4 * jj + 3] = __builtin_fmaf(d.w, blk[4 * jj + 3], acc[i][4 * jj + 3]);
+            }
+        }
+    };
+#pragma unroll
+    for (int c = 0; c < NC; c++) {
+        const int i = c >> 2, g = c & 3;
+        __builtin_amdgcn_sched_barrier(0);
+        uint32_t A[12];   // the operands of h and l, six dwords each
+#pragma unroll
+        for (int j = 0; j < 3; j++) {
+            const int q = 3 * g + j;
+            const uint4 v = *(const uint4 *)(act_lds + aofs[q & 3] + (q >> 2) * PF_CHUNK + i * 32u * 128u);
+            A[4 * j] = v.x; A[4 * j + 1] = v.y; A[4 * j + 2] = v.z; A[4 * j + 3] = v.w;
+        }
+        if (g == 0) G = *(const uint4 *)(gs_lds + 16u * (32u * i + col));
+        // -zp * gsum: two groups' sums are one operand, the other group's
+        // zero point is zero
+        typedef uint32_t u2 __attribute__((ext_vector_type(2)));
+        const u2 ga = g < 2 ? u2{G.x, G.y} : u2{G.z, G.w};
+        const u2 zb = (g & 1) ? u2{0u, b.z[g]} : u2{b.z[g], 0u};
+        f16v d = {0.0f};
+        d = __builtin_amdgcn_mfma_f32_32x32x8f16(__builtin_bit_cast(h4v, ga), __builtin_bit_cast(h4v, zb), d, 0, 0, 0);
+        d = pf_mfma6<FMT_E3M2>(A, b.w[g], d);
+        D[c & 1] = pf_mfma6<FMT_E2M3>(A + 6, b.w[g], d);
+        if (c > 0) finish(c - 1);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    finish(NC - 1);
 }
 
 // The tile's outputs.  D layout: lane holds column col, tokens
 // 8*(r/4) + 4*kh + r%4.  Gate/up: mid = ((g*sig(g))*u)*w per pair; down:
 // the per-pair rows.
 template <bool Q3, int NTB>
-__device__ __forceinline__ void pf_epilogue(const pf_params &p, const float (*acc)[16], const uint32_t *s_pair,
+__device__ __forceinline__ void pf_epilogue(const pf_params &p, const f16v *acc, const uint32_t *s_pair,
                                             const float *s_w, const uint64_t *s_tab, uint32_t kh, uint32_t col,
                                             uint32_t wcol, uint32_t cnt) {
 #pragma unroll
@@ -632,114 +573,128 @@ __device__ __forceinline__ void pf_epilogue(const pf_params &p, const float (*ac
 // epilogue mid = ((g*sig(g))*u)*w per pair.  Down (Q3 = false): row tile =
 // 128 output rows, 32 per wave; epilogue down_pair[pair][row].  One item
 // (tile, row tile) per workgroup: tiles interleaved over the XCDs, a tile's
-// row tiles consecutive on one.  (A persistent form, each workgroup taking
-// every G-th item and issuing the next item's first loads before the
-// current item's epilogue, measured slower: down 652 -> 677 us at config 3
-// with 40 more VGPRs; gate/up did not fit its registers.)
+// row tiles consecutive on one.
+//
+// Pipeline: at the top of a block its weight words (registers) and its
+// activations (LDS) have landed; the words are dequantised at once, then the
+// next block's activations go into the other buffer and the words of the
+// block after next into the same registers while this block's chains run.
+// The activations are issued first, so that waiting for them leaves the
+// newest weight words in flight.
+template <bool Q3, int NTB, typename ISSUE>
+__device__ __forceinline__ void pf_loop(const uint8_t *wrow, uint32_t nblk, ISSUE &&issue_act,
+                                        const uint8_t (*s_act)[PF_ACT_BUF], const uint8_t (*s_gs)[16u * PF_T],
+                                        const float (*s_d)[PF_T], uint32_t kh, uint32_t col,
+                                        pf_raw_t<Q3, false> &even, pf_raw_t<Q3, true> &oddr,
+                                        f16v *acc) {
+#pragma unroll
+    for (int i = 0; i < NTB; i++)
+#pragma unroll
+        for (int r2 = 0; r2 < 16; r2++) acc[i][r2] = 0.0f;
+    uint32_t aofs[4];
+#pragma unroll
+    for (uint32_t m = 0; m < 4u; m++) aofs[m] = 128u * col + 16u * ((2u * m) ^ kh ^ (col & 7u));
+    const uint32_t zt[2] = {kh ? 0u : 0x42403C00u, kh ? 0u : 0x47464544u};
+    constexpr std::integral_constant<bool, false> no{};
+    constexpr std::integral_constant<bool, true> yes{};
+    // next: block b + 1 exists; next2: b + 2 too
+    auto step = [&](uint32_t b, auto &raw, auto odd, auto next, auto next2) {
+        constexpr int P = decltype(odd)::value ? 1 : 0;
+        if constexpr (decltype(next)::value) wait_vm_keep_weights<Q3>();
+        else wait_vm0();
+        raw_ready(raw);
+        __syncthreads();
+        pf_b w;
+        if constexpr (Q3) pf_dequant<true, P ? 16 : 0>(w, raw, zt);
+        else pf_dequant<false, 0>(w, pf_words(raw), zt);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (decltype(next)::value) issue_act(b + 1u, NTB);
+        if constexpr (decltype(next2)::value) pf_wload<Q3, P>(raw, wrow, b + 2u, kh);
+        pf_block<NTB>(w, s_act[P], s_gs[P], s_d[P], aofs, kh, col, acc);
+    };
+    uint32_t b = 0;
+#pragma clang loop unroll(disable)
+    for (; b + 3u < nblk; b += 2u) {
+        step(b, even, no, yes, yes);
+        step(b + 1u, oddr, yes, yes, yes);
+    }
+    if (b + 2u == nblk) {
+        step(b, even, no, yes, no);
+        step(b + 1u, oddr, yes, no, no);
+    } else {
+        if (b + 3u == nblk) {
+            step(b, even, no, yes, yes);
+            step(b + 1u, oddr, yes, yes, no);
+            b += 2u;
+        }
+        step(b, even, no, no, no);
+    }
+}
+
 template <bool Q3>
-__global__ void __launch_bounds__(pf_cfg<Q3>::NW * 64, Q3 ? 1 : 2) pf_expert_kernel(pf_params p) {
-    constexpr uint32_t NW = pf_cfg<Q3>::NW, NBUF = pf_cfg<Q3>::NBUF;
-    __shared__ __align__(16) uint8_t s_act[NBUF][PF_ACT_BUF];
-    __shared__ __align__(16) float s_cd[NBUF][PF_CD_ROWS * PF_T];
+__global__ void __launch_bounds__(PF_NW * 64, 2) pf_expert_kernel(pf_params p) {
+    __shared__ __align__(16) uint8_t s_act[2][PF_ACT_BUF];
+    __shared__ __align__(16) uint8_t s_gs[2][16u * PF_T];   // [slot][group]
+    __shared__ __align__(16) float s_d[2][PF_T];
     __shared__ uint32_t s_pair[PF_T];
     __shared__ float s_w[PF_T];
     __shared__ uint64_t s_tab[Q3 ? 32 : 1];    // the exp table of the SwiGLU epilogue
+    const uint32_t idx = blockIdx.x, xcd = idx & 7u, item = idx >> 3;
+    const uint32_t t = xcd + 8u * (item / p.n_rt), rt = item % p.n_rt;
+    if (t >= p.tiles[0]) return;
     const uint32_t tid = threadIdx.x, lane = tid & 63u, kh = lane >> 5, col = lane & 31u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t nblk = p.nblk;
-    // activation rows: tile slot `lane` for the tables; slot 32*gi + lane%32
-    // for the codes (pad slots repeat the last pair).  8 waves: wave 4*gi + wq
-    // copies slot group gi; 4 waves: wave wq copies both groups.
-    constexpr uint32_t NG = NW == 8u ? 1u : 2u;      // slot groups a wave copies
-    constexpr int NJ = 4 * (int)NG;
-    const uint32_t wq = wave & 3u;
-    const uint32_t act_l = lds_addr(&s_act[0][0]), cd_l = lds_addr(&s_cd[0][0]);
-    const uint32_t blk_bytes = Q3 ? SF37_Q3_BYTES : SF37_Q2_BYTES;
-    const uint64_t row_bytes = (uint64_t)nblk * blk_bytes;
-    // codes: a wave loads slot pairs (t, t + 16), t = 4q .. 4q+3 of its slot
-    // group(s): lanes 0..31 read slot t's 512-byte row, lanes 32..63 slot
-    // t + 16's.  Each load's per-lane byte offset within a block's codes is
-    // the same for every block: the 8-wave kernel forms its four once
-    // (measured 1-3 % faster); the 4-wave kernel re-forms its eight per
-    // block (eight more VGPRs measured 2 % slower there)
-    auto lane_off = [&](const pf_item<Q3> &it, int jj) -> uint32_t {
-        const uint32_t k = (uint32_t)jj >> 2, t = 4u * wq + ((uint32_t)jj & 3u);
-        const uint32_t r0 = (uint32_t)__builtin_amdgcn_readlane((int)it.rowoff_c[k], (int)t);
-        const uint32_t r1 = (uint32_t)__builtin_amdgcn_readlane((int)it.rowoff_c[k], (int)t + 16);
-        return (kh ? r1 : r0) + 16u * col;
-    };
-    // the workgroup's item (tile, row tile), its pairs and routing weights
-    // in s_pair / s_w
-    pf_item<Q3> it;
-    {
-        const uint32_t idx = blockIdx.x, xcd = idx & 7u, slot = idx >> 3;
-        const uint32_t t = xcd + 8u * (slot / p.n_rt), rt = slot % p.n_rt;
-        if (t >= p.tiles[0]) return;
-        const uint4 ti = ((const uint4 *)p.tiles)[1 + t];
-        it.e = ti.x;
-        it.p0 = ti.y;
-        it.cnt = ti.z;
-        it.ntb = (it.cnt + 31u) / 32u;
-        if (tid < PF_T) {
-            const uint32_t pr = p.sorted[it.p0 + (tid < it.cnt ? tid : it.cnt - 1u)];
-            s_pair[tid] = pr;
-            if (Q3) s_w[tid] = p.weights[pr];
-        }
-#pragma unroll
-        for (uint32_t g = 0; g < NG; g++) {
-            const uint32_t gi = NW == 8u ? wave >> 2 : g;
-            const uint32_t sl = 32u * gi + (lane & 31u);
-            const uint32_t pr = p.sorted[it.p0 + (sl < it.cnt ? sl : it.cnt - 1u)];
-            it.rowoff_c[g] = (Q3 ? pr / p.topk : pr) * nblk * (SF37_QK * 2u);
-        }
-        if constexpr (NW == 8u) {
-#pragma unroll
-            for (int jj = 0; jj < NJ; jj++) it.voff[jj] = lane_off(it, jj);
-        }
-        // this lane's weight row
-        it.wcol = Q3 ? rt * PF_GU_R + 16u * wave + (col & 15u) : rt * PF_DN_R + 32u * wave + col;
-        it.wrow = (Q3 && col >= 16u ? p.w1 : p.w0) + ((uint64_t)it.e * p.out_rows + it.wcol) * row_bytes;
+    const uint4 ti = ((const uint4 *)p.tiles)[1 + t];
+    const uint32_t e = ti.x, p0 = ti.y, cnt = ti.z;
+    // this lane's weight row; block 0's words start loading, block 1's after
+    // the first activations
+    const uint32_t wcol = Q3 ? rt * PF_GU_R + 16u * wave + (col & 15u) : rt * PF_DN_R + 32u * wave + col;
+    const uint8_t *wrow = (Q3 && col >= 16u ? p.w1 : p.w0) +
+                          ((uint64_t)e * p.out_rows + wcol) * ((uint64_t)nblk * (Q3 ? SF37_Q3_BYTES : SF37_Q2_BYTES));
+    pf_raw_t<Q3, false> even;
+    pf_raw_t<Q3, true> oddr;
+    pf_wload<Q3, false>(even, wrow, 0, kh);
+    // pair of tile slot sl (pad slots repeat the last pair) and its activation row
+    auto slot_pair = [&](uint32_t sl) { return p.sorted[p0 + (sl < cnt ? sl : cnt - 1u)]; };
+    auto slot_row = [&](uint32_t pr) { return (Q3 ? pr / p.topk : pr) * nblk; };
+    const uint32_t mine = slot_pair(lane);
+    if (tid < PF_T) {
+        s_pair[tid] = mine;
+        if (Q3) s_w[tid] = p.weights[mine];
     }
     if (Q3) sf37_stage_exp_tab(s_tab);          // read after the block loop's barriers
-    // slice `part` of `nparts` (compile-time after inlining) of block b's
-    // activation loads
-    auto issue_act = [&](uint32_t b, int part, int nparts) {
-        const uint32_t bf = b % NBUF;
-        const uint8_t *cb = (const uint8_t *)p.act + (uint64_t)b * (SF37_QK * 2u);
-        const int j0 = NJ * part / nparts, j1 = NJ * (part + 1) / nparts;
+    // activation loads: wave w copies slot octets w and w + 4 (one per
+    // 32-pair block): lane l reads piece (l % 8) ^ (l / 8) of a chunk of slot
+    // l / 8; wave 0 also the group sums, wave 1 the scales, a lane per slot
+    uint32_t voff[2];
 #pragma unroll
-        for (int jj = j0; jj < j1; jj++) {
-            const uint32_t k = (uint32_t)jj >> 2, gi = NW == 8u ? wave >> 2 : k;
-            const uint32_t t = 4u * wq + ((uint32_t)jj & 3u);
-            uint32_t vo;
-            if constexpr (NW == 8u) vo = it.voff[jj];
-            else vo = lane_off(it, jj);
-            lds_dma16(act_l + bf * PF_ACT_BUF + gi * PF_GRP + t * PF_RS, vo, cb);
-        }
-        if (part == 0) {   // tables of all slots: row a = C_a (a < 4) or d (a = 4).  8 waves:
-                           // wave a < 5 loads row a, waves 5..7 row 4 again; 4 waves: wave w
-                           // loads rows w and 4 (the same bytes from every wave; no branch)
+    for (uint32_t k = 0; k < 2u; k++)
+        voff[k] = slot_row(slot_pair(8u * (wave + 4u * k) + (lane >> 3))) * PF_BLK + 16u * ((lane & 7u) ^ (lane >> 3));
+    const uint32_t srow = slot_row(mine);
+    const uint32_t act_l = lds_addr(&s_act[0][0]), gs_l = lds_addr(&s_gs[0][0]), d_l = lds_addr(&s_d[0][0]);
+    auto issue_act = [&](uint32_t b, uint32_t ntb) {
+        const uint32_t bf = b & 1u;
 #pragma unroll
-            for (uint32_t k = 0; k < (NW == 8u ? 1u : 2u); k++) {
-                const uint32_t a = NW == 8u ? (wave < 5u ? wave : 4u) : (k ? 4u : wave);
-                const float *tb = p.tab + ((uint64_t)b * 5u + a) * p.tab_stride + it.p0;
-                lds_dma4(cd_l + bf * (PF_CD_ROWS * PF_T * 4u) + (NW == 8u ? wave : a) * PF_T * 4u, 4u * lane, tb);
-            }
-        }
+        for (uint32_t k = 0; k < 2u; k++)
+            if (k < ntb)
+#pragma unroll
+                for (uint32_t c = 0; c < 3u; c++)
+                    lds_dma16(act_l + bf * PF_ACT_BUF + c * PF_CHUNK + (wave + 4u * k) * DMA16_SPAN, voff[k],
+                              p.act + (uint64_t)b * PF_BLK + c * 128u);
+        pf_rec_load(wave, gs_l + bf * DMA16_SPAN, d_l + bf * DMA4_SPAN, srow * PF_REC, p.rec + b * PF_REC);
     };
-    // the first loads: block 0's weights, its activation rows (and block 1's
-    // with three buffers)
-    pf_raw_t<Q3> ra;
-    issue_act(0, 0, 1);
-    pf_wload<Q3>(ra, it.wrow, 0, kh);
-    if constexpr (NBUF == 3u) issue_act(nblk > 1u ? 1u : 0u, 0, 1);
-    float acc[2][16];
-    if (it.ntb == 1) {
-        pf_loop<Q3, 1>(p, it.wrow, issue_act, s_act, s_cd, kh, col, ra, acc);
-        pf_epilogue<Q3, 1>(p, acc, s_pair, s_w, s_tab, kh, col, it.wcol, it.cnt);
+    f16v acc[2];
+    if (cnt <= 32u) {
+        issue_act(0, 1);
+        if (nblk > 1u) pf_wload<Q3, true>(oddr, wrow, 1u, kh);
+        pf_loop<Q3, 1>(wrow, nblk, issue_act, s_act, s_gs, s_d, kh, col, even, oddr, acc);
+        pf_epilogue<Q3, 1>(p, acc, s_pair, s_w, s_tab, kh, col, wcol, cnt);
     } else {
-        pf_loop<Q3, 2>(p, it.wrow, issue_act, s_act, s_cd, kh, col, ra, acc);
-        pf_epilogue<Q3, 2>(p, acc, s_pair, s_w, s_tab, kh, col, it.wcol, it.cnt);
+        issue_act(0, 2);
+        if (nblk > 1u) pf_wload<Q3, true>(oddr, wrow, 1u, kh);
+        pf_loop<Q3, 2>(wrow, nblk, issue_act, s_act, s_gs, s_d, kh, col, even, oddr, acc);
+        pf_epilogue<Q3, 2>(p, acc, s_pair, s_w, s_tab, kh, col, wcol, cnt);
     }
 }
 
@@ -1118,35 +1073,31 @@ extern "C" uint32_t sf37k_pf_max_tiles(uint32_t n_pairs, uint32_t max_groups) {
 
 extern "C" int sf37k_pf_supported(uint32_t in_dim, uint32_t mid_dim, uint32_t out_dim) {
     return in_dim % SF37_QK == 0 && mid_dim % SF37_QK == 0 && mid_dim % PF_GU_R == 0 &&
-           out_dim % PF_DN_R == 0 && in_dim > 0 && mid_dim > 0;   // 32 weight columns per wave
+           out_dim % PF_DN_R == 0 && in_dim > 0 && mid_dim > 0;
 }
 
-extern "C" int sf37k_pf_act(int q3, void *codes_v, float *tab, const float *x, uint32_t dim,
-                            uint32_t n_rows, sf37_stream_t s) {
-    _Float16 *codes = (_Float16 *)codes_v;
+// Activation operand buffer of n_rows rows: the fields, then the records.
+extern "C" uint64_t sf37k_pf_act_bytes(uint32_t dim, uint64_t n_rows) {
+    return (uint64_t)(dim / SF37_QK) * n_rows * (PF_BLK + PF_REC);
+}
+static uint8_t *pf_act_rec(const void *act, uint32_t nblk, uint64_t n_rows) {
+    return (uint8_t *)act + nblk * n_rows * PF_BLK;
+}
+
+extern "C" int sf37k_pf_act(int q3, void *act, const float *x, uint32_t dim, uint32_t n_rows, sf37_stream_t s) {
     const uint32_t nblk = dim / SF37_QK;
     const uint64_t units = (uint64_t)nblk * n_rows;
     if (units == 0) return 0;
     if (units > 0xffffffffu) return (int)hipErrorInvalidValue;
+    uint32_t *codes = (uint32_t *)act, *rec = (uint32_t *)pf_act_rec(act, nblk, n_rows);
     // four units per workgroup pass; at most 2048 workgroups, each wave then
     // walks several units
     const uint64_t wgs = (units + 3u) / 4u;
     const dim3 grid((unsigned)(wgs < 2048u ? wgs : 2048u));
     if (q3)
-        hipLaunchKernelGGL(pf_act_kernel<true>, grid, dim3(256), 0, (hipStream_t)s, codes, tab, x, nblk, n_rows);
+        hipLaunchKernelGGL(pf_act_kernel<true>, grid, dim3(256), 0, (hipStream_t)s, codes, rec, x, nblk, n_rows);
     else
-        hipLaunchKernelGGL(pf_act_kernel<false>, grid, dim3(256), 0, (hipStream_t)s, codes, tab, x, nblk, n_rows);
-    return (int)hipGetLastError();
-}
-
-extern "C" uint32_t sf37k_pf_tab_stride(uint32_t n_pairs) { return (n_pairs + PF_T + 63u) & ~63u; }
-
-extern "C" int sf37k_pf_tab_sort(float *tabs, const float *tab, const uint32_t *sorted_pairs, uint32_t n_pairs,
-                                 uint32_t dim, uint32_t div, sf37_stream_t s) {
-    const uint32_t nblk = dim / SF37_QK;
-    if (n_pairs == 0) return 0;
-    hipLaunchKernelGGL(pf_tab_sort_kernel, dim3((n_pairs + 255u) / 256u, nblk), dim3(256), 0, (hipStream_t)s, tabs,
-                       tab, sorted_pairs, n_pairs, nblk, div, sf37k_pf_tab_stride(n_pairs));
+        hipLaunchKernelGGL(pf_act_kernel<false>, grid, dim3(256), 0, (hipStream_t)s, codes, rec, x, nblk, n_rows);
     return (int)hipGetLastError();
 }
 
@@ -1156,47 +1107,47 @@ extern "C" int sf37k_pf_tiles(uint32_t *tiles, const uint32_t *group_info, uint3
     return (int)hipGetLastError();
 }
 
+static void pf_act_params(pf_params &p, const void *act, uint32_t dim, uint64_t n_rows) {
+    p.nblk = dim / SF37_QK;
+    p.act = (const uint8_t *)act;
+    p.rec = pf_act_rec(act, p.nblk, n_rows);
+}
+
 extern "C" int sf37k_pf_gate_up(float *mid, float *gate_out, float *up_out, const uint8_t *gate_w,
-                                const uint8_t *up_w, const void *act, const float *tab,
-                                const uint32_t *tiles, const uint32_t *sorted_pairs, const float *weights,
-                                uint32_t max_tiles, uint32_t tab_stride, uint32_t topk, uint32_t in_dim,
-                                uint32_t mid_dim, float clamp, sf37_stream_t s) {
+                                const uint8_t *up_w, const void *act, const uint32_t *tiles,
+                                const uint32_t *sorted_pairs, const float *weights, uint32_t max_tiles,
+                                uint32_t n_tok, uint32_t topk, uint32_t in_dim, uint32_t mid_dim, float clamp,
+                                sf37_stream_t s) {
     pf_params p = {};
     p.mid = mid;
     p.gate_out = gate_out;
     p.up_out = up_out;
     p.w0 = gate_w;
     p.w1 = up_w;
-    p.act = (const _Float16 *)act;
-    p.tab = tab;
+    pf_act_params(p, act, in_dim, n_tok);
     p.tiles = tiles;
     p.sorted = sorted_pairs;
     p.weights = weights;
     p.topk = topk;
-    p.nblk = in_dim / SF37_QK;
     p.out_rows = mid_dim;
     p.n_rt = mid_dim / PF_GU_R;
-    p.tab_stride = tab_stride;
     p.clamp = clamp;
-    hipLaunchKernelGGL(pf_expert_kernel<true>, dim3(pf_grid(max_tiles, p.n_rt)), dim3(pf_cfg<true>::NW * 64), 0, (hipStream_t)s, p);
+    hipLaunchKernelGGL(pf_expert_kernel<true>, dim3(pf_grid(max_tiles, p.n_rt)), dim3(PF_NW * 64), 0, (hipStream_t)s, p);
     return (int)hipGetLastError();
 }
 
-extern "C" int sf37k_pf_down(float *down_pair, const uint8_t *down_w, const void *act, const float *tab,
-                             const uint32_t *tiles, const uint32_t *sorted_pairs, uint32_t max_tiles,
-                             uint32_t tab_stride, uint32_t mid_dim, uint32_t out_dim, sf37_stream_t s) {
+extern "C" int sf37k_pf_down(float *down_pair, const uint8_t *down_w, const void *act, const uint32_t *tiles,
+                             const uint32_t *sorted_pairs, uint32_t max_tiles, uint32_t n_pairs, uint32_t mid_dim,
+                             uint32_t out_dim, sf37_stream_t s) {
     pf_params p = {};
     p.down_pair = down_pair;
     p.w0 = down_w;
-    p.act = (const _Float16 *)act;
-    p.tab = tab;
+    pf_act_params(p, act, mid_dim, n_pairs);
     p.tiles = tiles;
     p.sorted = sorted_pairs;
-    p.nblk = mid_dim / SF37_QK;
     p.out_rows = out_dim;
     p.n_rt = out_dim / PF_DN_R;
-    p.tab_stride = tab_stride;
-    hipLaunchKernelGGL(pf_expert_kernel<false>, dim3(pf_grid(max_tiles, p.n_rt)), dim3(pf_cfg<false>::NW * 64), 0, (hipStream_t)s, p);
+    hipLaunchKernelGGL(pf_expert_kernel<false>, dim3(pf_grid(max_tiles, p.n_rt)), dim3(PF_NW * 64), 0, (hipStream_t)s, p);
     return (int)hipGetLastError();
 }
 

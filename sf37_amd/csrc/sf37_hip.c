@@ -1072,13 +1072,9 @@ typedef struct {
     void *xq, *midq;
     uint32_t *ginfo, *sorted, *counts, *offsets, *hist;
     float *mid, *down_pair;
-    void *x16, *m16;        /* matrix-core path: fp16 codes in MFMA order */
-    float *xtab, *mtab;     /* their per-block tables */
-    float *xtabs, *mtabs;   /* the tables in dispatch order */
+    void *xact, *mact;      /* matrix-core path: rows and mid rows as MFMA operands */
     uint32_t *tiles;
 } routed_scratch;
-
-#define PF_TAB_BYTES 32u
 
 static uint64_t routed_layout(const routed_args *a, int slots, int pf, int need_mid, int need_down,
                               char *base, routed_scratch *s) {
@@ -1091,13 +1087,9 @@ static uint64_t routed_layout(const routed_args *a, int slots, int pf, int need_
         off = align256(off + (bytes));                                 \
     } while (0)
     if (pf) {
-        RESERVE(x16, void *, (uint64_t)a->n_tok * a->in_dim * 2u);
-        RESERVE(xtab, float *, (uint64_t)a->n_tok * (a->in_dim / QK) * PF_TAB_BYTES);
-        RESERVE(m16, void *, pairs * a->mid_dim * 2u);
-        RESERVE(mtab, float *, pairs * (a->mid_dim / QK) * PF_TAB_BYTES);
+        RESERVE(xact, void *, sf37k_pf_act_bytes(a->in_dim, a->n_tok));
+        RESERVE(mact, void *, sf37k_pf_act_bytes(a->mid_dim, pairs));
         RESERVE(tiles, uint32_t *, ((uint64_t)sf37k_pf_max_tiles((uint32_t)pairs, (uint32_t)groups) + 1u) * 16u);
-        RESERVE(xtabs, float *, (uint64_t)(a->in_dim / QK) * 5u * sf37k_pf_tab_stride((uint32_t)pairs) * 4u);
-        RESERVE(mtabs, float *, (uint64_t)(a->mid_dim / QK) * 5u * sf37k_pf_tab_stride((uint32_t)pairs) * 4u);
     } else {
         RESERVE(xq, void *, (uint64_t)a->n_tok * (a->in_dim / QK) * Q8KB);
         RESERVE(midq, void *, pairs * (a->mid_dim / QK) * Q8KB);
@@ -1160,33 +1152,28 @@ static int side_stream_ready(void) {
     return 1;
 }
 
-/* Matrix-core pipeline (k_prefill.hip): x to fp16 MFMA codes, dispatch,
- * tiles, gate/up + SwiGLU*w, mid to fp16 MFMA codes, down, combine. */
+/* Matrix-core pipeline (k_prefill.hip): x to MFMA operands, dispatch, tiles,
+ * gate/up + SwiGLU*w, mid to MFMA operands, down, combine. */
 static int routed_pf(const routed_args *a, const routed_scratch *s, float *out, float *mid, float *down_pair,
                      float *gate_out, float *up_out) {
     const sf37_stream_t st = (sf37_stream_t)g_stream;
     const uint32_t pairs = a->n_tok * a->topk;
     const uint32_t groups = a->n_expert;
     const uint32_t max_tiles = sf37k_pf_max_tiles(pairs, groups);
-    const uint32_t tstride = sf37k_pf_tab_stride(pairs);
-    return LAUNCH(SF37_HIP_STAGE_PF_ACT_X, sf37k_pf_act(1, s->x16, s->xtab, a->x, a->in_dim, a->n_tok, st),
+    return LAUNCH(SF37_HIP_STAGE_PF_ACT_X, sf37k_pf_act(1, s->xact, a->x, a->in_dim, a->n_tok, st),
                   "routed_moe mfma input codes launch") &&
            LAUNCH(SF37_HIP_STAGE_DISPATCH, sf37k_moe_dispatch(s->ginfo, s->sorted, s->counts, s->offsets, a->selected,
                                                               pairs, a->n_expert, s->hist, st),
                   "routed_moe dispatch launch") &&
            LAUNCH(SF37_HIP_STAGE_PF_TILES, sf37k_pf_tiles(s->tiles, s->ginfo, groups, st), "routed_moe tiles launch") &&
-           LAUNCH(SF37_HIP_STAGE_PF_TILES, sf37k_pf_tab_sort(s->xtabs, s->xtab, s->sorted, pairs, a->in_dim, a->topk, st),
-                  "routed_moe input tables launch") &&
-           LAUNCH(SF37_HIP_STAGE_PF_GATE_UP, sf37k_pf_gate_up(mid, gate_out, up_out, a->gate_w, a->up_w, s->x16, s->xtabs,
-                                                             s->tiles, s->sorted, a->weights, max_tiles, tstride,
+           LAUNCH(SF37_HIP_STAGE_PF_GATE_UP, sf37k_pf_gate_up(mid, gate_out, up_out, a->gate_w, a->up_w, s->xact,
+                                                             s->tiles, s->sorted, a->weights, max_tiles, a->n_tok,
                                                              a->topk, a->in_dim, a->mid_dim, a->clamp, st),
                   "routed_moe mfma gate/up launch") &&
-           LAUNCH(SF37_HIP_STAGE_PF_ACT_MID, sf37k_pf_act(0, s->m16, s->mtab, mid, a->mid_dim, pairs, st),
+           LAUNCH(SF37_HIP_STAGE_PF_ACT_MID, sf37k_pf_act(0, s->mact, mid, a->mid_dim, pairs, st),
                   "routed_moe mfma mid codes launch") &&
-           LAUNCH(SF37_HIP_STAGE_PF_ACT_MID, sf37k_pf_tab_sort(s->mtabs, s->mtab, s->sorted, pairs, a->mid_dim, 1u, st),
-                  "routed_moe mid tables launch") &&
-           LAUNCH(SF37_HIP_STAGE_PF_DOWN, sf37k_pf_down(down_pair, a->down_w, s->m16, s->mtabs, s->tiles, s->sorted,
-                                                       max_tiles, tstride, a->mid_dim, a->out_dim, st),
+           LAUNCH(SF37_HIP_STAGE_PF_DOWN, sf37k_pf_down(down_pair, a->down_w, s->mact, s->tiles, s->sorted, max_tiles,
+                                                       pairs, a->mid_dim, a->out_dim, st),
                   "routed_moe mfma down launch") &&
            routed_combine(a, out, down_pair);
 }

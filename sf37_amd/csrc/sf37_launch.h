@@ -116,29 +116,25 @@ int sf37k_synth_quant_rows(int type, uint8_t *dst, uint64_t row0, uint64_t nrows
 int sf37k_sigmoid_array(float *out, const float *x, uint64_t n, int mode, sf37_stream_t s);
 
 /* Routed experts on the matrix cores for many pairs per expert
- * (k_prefill.hip).  Activations are re-quantised to Q8_K and written as fp16
- * codes in the MFMA operand order of the weight format (q3 = 1: Q3 gate/up,
- * 0: Q2 down) with a table of 8 floats per (row, 256-block); groups are cut
- * into tiles of <= 128 pairs; gate/up and down read them.  codes: rows x dim
- * halves; tab: rows x dim/256 x 8 floats; tiles: (max_tiles + 1) x 4 words. */
+ * (k_prefill.hip).  Activations are re-quantised to Q8_K and written as
+ * 6-bit fields in the MFMA operand order of the weight format (q3 = 1: Q3
+ * gate/up, 0: Q2 down) with their group sums and scales, all in one buffer of
+ * sf37k_pf_act_bytes; groups are cut into tiles of <= 64 pairs; gate/up (rows
+ * = tokens) and down (rows = pairs) read them.  tiles: (max_tiles + 1) x 4
+ * words. */
 uint32_t sf37k_pf_max_tiles(uint32_t n_pairs, uint32_t max_groups);
 int sf37k_pf_supported(uint32_t in_dim, uint32_t mid_dim, uint32_t out_dim);
-int sf37k_pf_act(int q3, void *codes, float *tab, const float *x, uint32_t dim, uint32_t n_rows,
-                 sf37_stream_t s);
+uint64_t sf37k_pf_act_bytes(uint32_t dim, uint64_t n_rows);
+int sf37k_pf_act(int q3, void *act, const float *x, uint32_t dim, uint32_t n_rows, sf37_stream_t s);
 int sf37k_pf_tiles(uint32_t *tiles, const uint32_t *group_info, uint32_t max_groups, sf37_stream_t s);
-/* The per-block tables gathered into dispatch order (floats:
- * dim/256 x 5 x sf37k_pf_tab_stride(n_pairs)); row = pair / div. */
-uint32_t sf37k_pf_tab_stride(uint32_t n_pairs);
-int sf37k_pf_tab_sort(float *tabs, const float *tab, const uint32_t *sorted_pairs, uint32_t n_pairs, uint32_t dim,
-                      uint32_t div, sf37_stream_t s);
 int sf37k_pf_gate_up(float *mid, float *gate_out, float *up_out, const uint8_t *gate_w,
-                     const uint8_t *up_w, const void *act, const float *tab, const uint32_t *tiles,
+                     const uint8_t *up_w, const void *act, const uint32_t *tiles,
                      const uint32_t *sorted_pairs, const float *weights, uint32_t max_tiles,
-                     uint32_t tab_stride, uint32_t topk, uint32_t in_dim, uint32_t mid_dim, float clamp,
+                     uint32_t n_tok, uint32_t topk, uint32_t in_dim, uint32_t mid_dim, float clamp,
                      sf37_stream_t s);
-int sf37k_pf_down(float *down_pair, const uint8_t *down_w, const void *act, const float *tab,
-                  const uint32_t *tiles, const uint32_t *sorted_pairs, uint32_t max_tiles,
-                  uint32_t tab_stride, uint32_t mid_dim, uint32_t out_dim, sf37_stream_t s);
+int sf37k_pf_down(float *down_pair, const uint8_t *down_w, const void *act, const uint32_t *tiles,
+                  const uint32_t *sorted_pairs, uint32_t max_tiles, uint32_t n_pairs, uint32_t mid_dim,
+                  uint32_t out_dim, sf37_stream_t s);
 
 /* Shared expert (Q8_0) on the int8 matrix cores for many tokens
  * (k_prefill.hip): Q8_0 activations (a8: n_tok x dim int8 codes, xs: n_tok x
