@@ -252,7 +252,8 @@ void *sf37_hip_get_stream(void);
  *   "decode_select_in_up_max_tokens", "decode_up_dyn_pct", "decode_up_wgs",
  *   "decode_down_wgs"   decode tuning (results unchanged)
  *   "prefill_mfma"      1 (default): grouped batches run on the matrix cores;
- *   "prefill_min_pairs", "shared_min_tokens" the smallest batches that do
+ *   "prefill_min_pairs", "shared_min_tokens" the smallest batches that do;
+ *   "q8_0_min_tokens" the smallest batches of the Q8_0 products that do
  *   "shared_stream"     1 (default): a prefill batch's Q8_0 shared expert
  *                       runs on a second stream of the library (default
  *                       priority), forked after its input rows and joined

@@ -767,8 +767,8 @@ __global__ void __launch_bounds__(256) sh_act_kernel(int8_t *__restrict__ a8, fl
 }
 
 struct sh_params {
-    float *out0;                   // gate/up: mid (SwiGLU) [tok][rows]; down: out [tok][rows]
-    const uint8_t *w0, *w1;        // Q8_0 gate, up (or down) [rows][nb blocks]
+    float *out0, *out1;            // gate/up: mid (SwiGLU) [tok][rows]; else the products with w0 and w1 [tok][rows]
+    const uint8_t *w0, *w1;        // Q8_0 gate, up (or one or two matrices) [rows][nb blocks]
     const int8_t *act;             // [tok][nb * 32]
     const float *xs;               // [tok][nb]
     uint32_t n_tok, nb, rows, n_ct, n_tt;
@@ -956,8 +956,10 @@ __device__ __forceinline__ void sh_chunk_batched(const sh_raw &r, const uint8_t 
 }
 
 // GU: gate/up, 16 gate + 16 up rows per wave, epilogue mid = (g*sig(g))*u
-// (shared clamp).  Otherwise down: 32 output rows per wave, out written
-// directly.  TBW = 2: a wave takes both 32-token blocks of the tile, the
+// (shared clamp).  Otherwise plain products: 32 output rows per wave, written
+// directly (the last column tile may be partial: its missing columns repeat
+// the last row and are not stored); column tiles n_ct .. 2 n_ct - 1 are the
+// second matrix's.  TBW = 2: a wave takes both 32-token blocks of the tile, the
 // workgroup 128 weight columns; TBW = 1 (batches whose TBW = 2 grid would
 // leave CUs idle): waves 2 c and 2 c + 1 take token block 0 and 1 of the
 // same 32 columns, the workgroup 64 columns.  BAT (TBW = 1 only): the chunk
@@ -970,7 +972,8 @@ __global__ void __launch_bounds__(256, 2) sh_gemm_kernel(sh_params p) {
     __shared__ uint64_t s_tab[GU ? 32 : 1];    // the exp table of the SwiGLU epilogue
     static_assert(TBW == 1 || TBW == 2, "token blocks per wave");
     if (GU) sf37_stage_exp_tab(s_tab);          // read after the chunk loop's barriers
-    const uint32_t tt = blockIdx.x % p.n_tt, ct = blockIdx.x / p.n_tt;
+    const uint32_t tt = blockIdx.x % p.n_tt, cti = blockIdx.x / p.n_tt;
+    const uint32_t mat = !GU && cti >= p.n_ct ? 1u : 0u, ct = cti - mat * p.n_ct;
     const uint32_t tid = threadIdx.x, lane = tid & 63u, kh = lane >> 5, col = lane & 31u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t tb0 = TBW == 2 ? 0u : (wave & 1u), cg = TBW == 2 ? wave : wave >> 1;
@@ -979,8 +982,10 @@ __global__ void __launch_bounds__(256, 2) sh_gemm_kernel(sh_params p) {
     const uint32_t nb = p.nb, nchunk = nb / SH_CB;
     // this lane's weight row
     const uint32_t wcol = GU ? ct * (COLS / 2u) + 16u * cg + (col & 15u) : ct * COLS + 32u * cg + col;
-    const bool second = GU && col >= 16u;
-    const uint8_t *wrow = (second ? p.w1 : p.w0) + (uint64_t)wcol * nb * SF37_Q8_0_BYTES;
+    const bool second = GU ? col >= 16u : mat != 0u;
+    const uint32_t wr = GU || wcol < p.rows ? wcol : p.rows - 1u;
+    const uint8_t *wrow = (second ? p.w1 : p.w0) + (uint64_t)wr * nb * SF37_Q8_0_BYTES;
+    float *out = GU || !mat ? p.out0 : p.out1;
     // DMA: load L = 2 wave + k fills rows 8 L .. 8 L + 7; lane l writes row
     // 8 L + l / 8, slot l % 8, which holds piece (l % 8) ^ (l / 8) of it
     uint32_t voff[2];
@@ -1051,13 +1056,13 @@ __global__ void __launch_bounds__(256, 2) sh_gemm_kernel(sh_params p) {
                 const uint32_t r2 = up_lane ? (uint32_t)k + 8u : (uint32_t)k;
                 const float g = up_lane ? ob : va, u = up_lane ? vb : oa;
                 const uint32_t t = t0 + 32u * (tb0 + i) + 8u * (r2 >> 2) + 4u * kh + (r2 & 3u);
-                if (t < p.n_tok) p.out0[(uint64_t)t * p.rows + wcol] = sf37_swiglu_mid_t(g, u, 1.0f, p.clamp, s_tab);
+                if (t < p.n_tok) out[(uint64_t)t * p.rows + wcol] = sf37_swiglu_mid_t(g, u, 1.0f, p.clamp, s_tab);
             }
         } else {
 #pragma unroll
             for (int r2 = 0; r2 < 16; r2++) {
                 const uint32_t t = t0 + 32u * (tb0 + i) + 8u * (r2 >> 2) + 4u * kh + (r2 & 3);
-                if (t < p.n_tok) p.out0[(uint64_t)t * p.rows + wcol] = acc[i][r2];
+                if (t < p.n_tok && wcol < p.rows) out[(uint64_t)t * p.rows + wcol] = acc[i][r2];
             }
         }
     }
@@ -1212,26 +1217,40 @@ extern "C" int sf37k_sh_gate_up(float *mid, const uint8_t *gate_w, const uint8_t
     return (int)hipGetLastError();
 }
 
-extern "C" int sf37k_sh_down(float *out, const uint8_t *down_w, const void *a8, const float *xs, uint32_t n_tok,
-                             uint32_t mid_dim, uint32_t out_dim, sf37_stream_t s) {
+extern "C" int sf37k_sh_matmul_supported(uint64_t in_dim, uint64_t out_dim, uint64_t n_tok) {
+    return in_dim > 0 && in_dim % (32u * SH_CB * 2u) == 0 && out_dim > 0 && out_dim < (1u << 24) && n_tok > 0 &&
+           n_tok * in_dim < (1ull << 32) && (out_dim + 63u) / 64u * 2u * ((n_tok + SH_T - 1u) / SH_T) < (1ull << 31);
+}
+
+extern "C" int sf37k_sh_matmul(float *out0, float *out1, const uint8_t *w0, const uint8_t *w1, const void *a8,
+                               const float *xs, uint32_t n_tok, uint32_t in_dim, uint32_t out_dim, sf37_stream_t s) {
     sh_params p = {};
-    p.out0 = out;
-    p.w0 = down_w;
+    p.out0 = out0;
+    p.out1 = out1;
+    p.w0 = w0;
+    p.w1 = w1;
     p.act = (const int8_t *)a8;
     p.xs = xs;
     p.n_tok = n_tok;
-    p.nb = mid_dim / 32u;
+    p.nb = in_dim / 32u;
     p.rows = out_dim;
     p.n_tt = (n_tok + SH_T - 1u) / SH_T;
-    if (sh_narrow(out_dim / 128u, p.n_tt)) {
-        p.n_ct = out_dim / 64u;
-        if (sh_batched(p.n_ct, p.n_tt))
-            hipLaunchKernelGGL((sh_gemm_kernel<false, 1, true>), dim3(p.n_ct * p.n_tt), dim3(256), 0, (hipStream_t)s, p);
+    const uint32_t mats = out1 ? 2u : 1u;
+    if (sh_narrow(mats * ((out_dim + 127u) / 128u), p.n_tt)) {
+        p.n_ct = (out_dim + 63u) / 64u;
+        const dim3 grid(mats * p.n_ct * p.n_tt);
+        if (sh_batched(mats * p.n_ct, p.n_tt))
+            hipLaunchKernelGGL((sh_gemm_kernel<false, 1, true>), grid, dim3(256), 0, (hipStream_t)s, p);
         else
-            hipLaunchKernelGGL((sh_gemm_kernel<false, 1>), dim3(p.n_ct * p.n_tt), dim3(256), 0, (hipStream_t)s, p);
+            hipLaunchKernelGGL((sh_gemm_kernel<false, 1>), grid, dim3(256), 0, (hipStream_t)s, p);
     } else {
-        p.n_ct = out_dim / 128u;
-        hipLaunchKernelGGL((sh_gemm_kernel<false, 2>), dim3(p.n_ct * p.n_tt), dim3(256), 0, (hipStream_t)s, p);
+        p.n_ct = (out_dim + 127u) / 128u;
+        hipLaunchKernelGGL((sh_gemm_kernel<false, 2>), dim3(mats * p.n_ct * p.n_tt), dim3(256), 0, (hipStream_t)s, p);
     }
     return (int)hipGetLastError();
+}
+
+extern "C" int sf37k_sh_down(float *out, const uint8_t *down_w, const void *a8, const float *xs, uint32_t n_tok,
+                             uint32_t mid_dim, uint32_t out_dim, sf37_stream_t s) {
+    return sf37k_sh_matmul(out, NULL, down_w, NULL, a8, xs, n_tok, mid_dim, out_dim, s);
 }

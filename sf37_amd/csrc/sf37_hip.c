@@ -56,6 +56,7 @@ static int64_t g_opt_down_combine = 1;
 static int64_t g_opt_prefill = 1;
 static int64_t g_opt_prefill_min_pairs = 256;
 static int64_t g_opt_shared_min_tok = 64;
+static int64_t g_opt_q8_0_min_tok = 20;
 static int64_t g_opt_shared_stream = 1;
 static int64_t g_opt_shared_slot = 1;
 /* the shared expert's side stream (default priority) and its fork / join
@@ -384,6 +385,7 @@ int sf37_hip_set_option(const char *name, int64_t value) {
     else if (!strcmp(name, "prefill_mfma")) g_opt_prefill = value ? 1 : 0;
     else if (!strcmp(name, "prefill_min_pairs")) g_opt_prefill_min_pairs = value < 0 ? 0 : value;
     else if (!strcmp(name, "shared_min_tokens")) g_opt_shared_min_tok = value < 0 ? 0 : value;
+    else if (!strcmp(name, "q8_0_min_tokens")) g_opt_q8_0_min_tok = value < 0 ? 0 : value;
     else if (!strcmp(name, "shared_stream")) g_opt_shared_stream = value ? 1 : 0;
     else if (!strcmp(name, "decode_shared_slot")) g_opt_shared_slot = value ? 1 : 0;
     else return 0;
@@ -405,6 +407,7 @@ int64_t sf37_hip_get_option(const char *name) {
     if (!strcmp(name, "prefill_mfma")) return g_opt_prefill;
     if (!strcmp(name, "prefill_min_pairs")) return g_opt_prefill_min_pairs;
     if (!strcmp(name, "shared_min_tokens")) return g_opt_shared_min_tok;
+    if (!strcmp(name, "q8_0_min_tokens")) return g_opt_q8_0_min_tok;
     if (!strcmp(name, "shared_stream")) return g_opt_shared_stream;
     if (!strcmp(name, "decode_shared_slot")) return g_opt_shared_slot;
     return -1;
@@ -744,6 +747,8 @@ int sf37_hip_swiglu_f32(sf37_hip_tensor *out, const sf37_hip_tensor *gate, const
 /* Q8_0 (sf37_cuda.cu:3319-3781, 6405-6440, 6649-6916)                       */
 /* ------------------------------------------------------------------------ */
 
+#define Q8_0_MFMA_MIN_OUTS 24576u
+
 static int q8_0_run(float *out0, float *out1, const uint8_t *w0, const uint8_t *w1, uint64_t in_dim,
                     uint64_t out_dim, const float *x, uint64_t n_tok) {
     const uint64_t nb = (in_dim + 31u) / 32u;
@@ -753,6 +758,22 @@ static int q8_0_run(float *out0, float *out1, const uint8_t *w0, const uint8_t *
     if (!s) return 0;
     int8_t *xq = (int8_t *)s;
     float *xs = (float *)(s + xq_bytes);
+    /* many tokens on the matrix cores (k_prefill.hip), same bits.  Their time
+     * hardly depends on the batch up to 256 tokens (a workgroup's chain over
+     * in_dim: 35 us at 4096, 12.5 at 1280), the dot kernel's grows with every
+     * output: measured (dot / matrix cores, us) 4096 -> 2 x 1280: 24 tokens
+     * 55 / 35, 777 about 1500 / 80, 2048 3981 / 128; 1280 -> 4096: 17 tokens
+     * 11.7 / 12.6, 24 14.2 / 12.5, 2048 537 / 60; 4096 -> 288: 64 tokens 31 /
+     * 37, 96 42 / 37, 2048 581 / 42. */
+    const uint64_t outs = n_tok * out_dim * (out1 ? 2u : 1u);
+    if (g_opt_prefill && n_tok >= (uint64_t)g_opt_q8_0_min_tok && outs >= Q8_0_MFMA_MIN_OUTS &&
+        sf37k_sh_matmul_supported(in_dim, out_dim, n_tok) &&
+        ((uintptr_t)w0 & 3u) == 0 && ((uintptr_t)w1 & 3u) == 0 && ((uintptr_t)x & 15u) == 0)
+        return LAUNCH(SF37_HIP_STAGE_Q8_0_ACT, sf37k_sh_act(xq, xs, x, (uint32_t)in_dim, (uint32_t)n_tok, (sf37_stream_t)g_stream),
+                      "q8_0 activations launch") &&
+               LAUNCH(SF37_HIP_STAGE_Q8_0_GEMM, sf37k_sh_matmul(out0, out1, w0, w1, xq, xs, (uint32_t)n_tok, (uint32_t)in_dim,
+                                                                (uint32_t)out_dim, (sf37_stream_t)g_stream),
+                      "q8_0 matrix-core matmul launch");
     if (!LAUNCH(SF37_HIP_STAGE_Q8_0_ACT, sf37k_q8_0_quantize(xq, xs, x, in_dim, n_tok, (sf37_stream_t)g_stream), "q8_0 quantize launch"))
         return 0;
     return LAUNCH(SF37_HIP_STAGE_Q8_0_GEMM, sf37k_q8_0_matmul(out0, out1, w0, w1, xq, xs, in_dim, out_dim, n_tok, (sf37_stream_t)g_stream),

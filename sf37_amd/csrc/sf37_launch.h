@@ -147,6 +147,11 @@ int sf37k_sh_gate_up(float *mid, const uint8_t *gate_w, const uint8_t *up_w, con
                      uint32_t n_tok, uint32_t in_dim, uint32_t mid_dim, float clamp, sf37_stream_t s);
 int sf37k_sh_down(float *out, const uint8_t *down_w, const void *a8, const float *xs, uint32_t n_tok,
                   uint32_t mid_dim, uint32_t out_dim, sf37_stream_t s);
+/* Q8_0 products of many tokens on the same kernels: out0 = w0 x, and with
+ * out1 also out1 = w1 x, from sf37k_sh_act's activations.  Any out_dim. */
+int sf37k_sh_matmul_supported(uint64_t in_dim, uint64_t out_dim, uint64_t n_tok);
+int sf37k_sh_matmul(float *out0, float *out1, const uint8_t *w0, const uint8_t *w1, const void *a8, const float *xs,
+                    uint32_t n_tok, uint32_t in_dim, uint32_t out_dim, sf37_stream_t s);
 
 /* Fused decode layer (up to 16 tokens): route, select, up, mid, down,
  * combine (k_decode.hip).  Pointers are device addresses; flags select the parts
