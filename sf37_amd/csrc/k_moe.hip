@@ -483,7 +483,8 @@ template <int MODE>
 __device__ __forceinline__ void combine_store(float *out, const float *base, float *resid, uint64_t i, float v) {
     if constexpr (MODE == 0) out[i] = v;
     else if constexpr (MODE == 1) out[i] = base[i] + v;
-    else resid[i] = resid[i] + (base[i] + v);
+    else if constexpr (MODE == 2) resid[i] = resid[i] + (base[i] + v);
+    else resid[i] = resid[i] + v;
 }
 
 template <int MODE>
@@ -533,6 +534,9 @@ __global__ void __launch_bounds__(256) combine4_kernel(float *out, const float *
     } else if constexpr (MODE == 1) {
         const float4 bv = *(const float4 *)(base + i);
         *(float4 *)(out + i) = make_float4(bv.x + acc.x, bv.y + acc.y, bv.z + acc.z, bv.w + acc.w);
+    } else if constexpr (MODE == 3) {
+        const float4 rv = *(const float4 *)(resid + i);
+        *(float4 *)(resid + i) = make_float4(rv.x + acc.x, rv.y + acc.y, rv.z + acc.z, rv.w + acc.w);
     } else {
         const float4 bv = *(const float4 *)(base + i), rv = *(const float4 *)(resid + i);
         *(float4 *)(resid + i) = make_float4(rv.x + (bv.x + acc.x), rv.y + (bv.y + acc.y), rv.z + (bv.z + acc.z),
@@ -650,6 +654,31 @@ extern "C" int sf37k_moe_dispatch(uint32_t *group_info, uint32_t *sorted_pairs, 
     return (int)hipGetLastError();
 }
 
+// One more slot per token: the shared expert as expert id n_expert with
+// weight 1.
+__global__ void __launch_bounds__(256) append_shared_kernel(int32_t *__restrict__ sel_out, float *__restrict__ w_out,
+                                                            const int32_t *__restrict__ sel,
+                                                            const float *__restrict__ w, uint32_t topk,
+                                                            uint32_t n_expert, uint32_t n) {
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    if (i >= n) return;
+    const uint32_t t = i / (topk + 1u), s = i - t * (topk + 1u);
+    const bool shared = s == topk;
+    const uint32_t e = shared ? n_expert : (uint32_t)sel[t * topk + s];
+    // an id out of range acts as expert 0, also one that names the added slot
+    sel_out[i] = (int32_t)(!shared && e >= n_expert ? 0u : e);
+    w_out[i] = shared ? 1.0f : w[t * topk + s];
+}
+
+extern "C" int sf37k_moe_append_shared(int32_t *sel_out, float *w_out, const int32_t *sel, const float *w,
+                                       uint32_t topk, uint32_t n_expert, uint32_t n_tok, sf37_stream_t s) {
+    const uint32_t n = n_tok * (topk + 1u);
+    if (n == 0) return 0;
+    hipLaunchKernelGGL(append_shared_kernel, dim3((n + 255u) / 256u), dim3(256), 0, (hipStream_t)s, sel_out, w_out,
+                       sel, w, topk, n_expert, n);
+    return (int)hipGetLastError();
+}
+
 extern "C" int sf37k_moe_slots(uint32_t *group_info, uint32_t *sorted_pairs, const int32_t *selected,
                                uint32_t topk, uint32_t n_expert, sf37_stream_t s) {
     hipLaunchKernelGGL(slots_kernel, dim3(1), dim3(64), 0, (hipStream_t)s, group_info, sorted_pairs,
@@ -698,8 +727,7 @@ extern "C" int sf37k_moe_combine(float *out, const float *down_pair, const float
                                  uint32_t topk, uint32_t out_dim, uint32_t n_tok, sf37_stream_t s) {
     const uint64_t n = (uint64_t)out_dim * n_tok;
     if (n == 0) return 0;
-    const int mode = resid ? 2 : (base ? 1 : 0);
-    if ((resid || base) && !base) return (int)hipErrorInvalidValue;
+    const int mode = resid ? (base ? 2 : 3) : (base ? 1 : 0);
     const bool vec = out_dim % 4u == 0 && topk >= 1u && topk <= 16u &&
                      (((uintptr_t)down_pair | (uintptr_t)out | (uintptr_t)base | (uintptr_t)resid) & 15u) == 0;
     const dim3 grid((unsigned)(((vec ? n / 4u : n) + 255) / 256));
@@ -709,17 +737,22 @@ extern "C" int sf37k_moe_combine(float *out, const float *down_pair, const float
         if (topk == 8u)                                                                                       \
             hipLaunchKernelGGL((combine4_kernel<M, 8>), grid, dim3(256), 0, (hipStream_t)s, out, down_pair, base, \
                                resid, topk, out_dim, n_tok);                                                  \
+        else if (topk == 9u)                                                                                  \
+            hipLaunchKernelGGL((combine4_kernel<M, 9>), grid, dim3(256), 0, (hipStream_t)s, out, down_pair, base, \
+                               resid, topk, out_dim, n_tok);                                                  \
         else                                                                                                  \
             hipLaunchKernelGGL((combine4_kernel<M, 0>), grid, dim3(256), 0, (hipStream_t)s, out, down_pair, base, \
                                resid, topk, out_dim, n_tok);                                                  \
     } while (0)
         if (mode == 0) SF37_COMBINE4(0);
         else if (mode == 1) SF37_COMBINE4(1);
-        else SF37_COMBINE4(2);
+        else if (mode == 2) SF37_COMBINE4(2);
+        else SF37_COMBINE4(3);
 #undef SF37_COMBINE4
     } else {
         if (mode == 0) hipLaunchKernelGGL(combine_kernel<0>, grid, dim3(256), 0, (hipStream_t)s, out, down_pair, base, resid, topk, out_dim, n_tok);
         else if (mode == 1) hipLaunchKernelGGL(combine_kernel<1>, grid, dim3(256), 0, (hipStream_t)s, out, down_pair, base, resid, topk, out_dim, n_tok);
+        else if (mode == 3) hipLaunchKernelGGL(combine_kernel<3>, grid, dim3(256), 0, (hipStream_t)s, out, down_pair, base, resid, topk, out_dim, n_tok);
         else hipLaunchKernelGGL(combine_kernel<2>, grid, dim3(256), 0, (hipStream_t)s, out, down_pair, base, resid, topk, out_dim, n_tok);
     }
     return (int)hipGetLastError();

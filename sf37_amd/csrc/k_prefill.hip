@@ -312,6 +312,9 @@ struct pf_params {
     const float *weights;
     uint32_t topk, nblk, out_rows, n_rt;
     float clamp;
+    const uint8_t *s0, *s1;        // the same of expert sh_id, which has tensors of its own
+    uint32_t sh_id;
+    float sh_clamp;
 };
 
 // Weight bytes of one lane for one Q3 block: the header dwords (scales, zero
@@ -534,7 +537,7 @@ __device__ __forceinline__ void pf_block(const pf_b &b, const uint8_t *act_lds, 
 // 8*(r/4) + 4*kh + r%4.  Gate/up: mid = ((g*sig(g))*u)*w per pair; down:
 // the per-pair rows.
 template <bool Q3, int NTB>
-__device__ __forceinline__ void pf_epilogue(const pf_params &p, const f16v *acc, const uint32_t *s_pair,
+__device__ __forceinline__ void pf_epilogue(const pf_params &p, float clamp, const f16v *acc, const uint32_t *s_pair,
                                             const float *s_w, const uint64_t *s_tab, uint32_t kh, uint32_t col,
                                             uint32_t wcol, uint32_t cnt) {
 #pragma unroll
@@ -553,7 +556,7 @@ __device__ __forceinline__ void pf_epilogue(const pf_params &p, const f16v *acc,
                 const uint32_t tl = 32u * i + 8u * ((uint32_t)r2 >> 2) + 4u * kh + ((uint32_t)r2 & 3u);
                 if (tl < cnt) {
                     const uint64_t at = (uint64_t)s_pair[tl] * p.out_rows + wcol;
-                    p.mid[at] = sf37_swiglu_mid_t(g, u, s_w[tl], p.clamp, s_tab);
+                    p.mid[at] = sf37_swiglu_mid_t(g, u, s_w[tl], clamp, s_tab);
                     if (p.gate_out) p.gate_out[at] = g;
                     if (p.up_out) p.up_out[at] = u;
                 }
@@ -646,11 +649,13 @@ __global__ void __launch_bounds__(PF_NW * 64, 2) pf_expert_kernel(pf_params p) {
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t nblk = p.nblk;
     const uint4 ti = ((const uint4 *)p.tiles)[1 + t];
-    const uint32_t e = ti.x, p0 = ti.y, cnt = ti.z;
+    const bool sh = ti.x == p.sh_id;
+    const uint32_t e = sh ? 0u : ti.x, p0 = ti.y, cnt = ti.z;
+    const uint8_t *w0 = sh ? p.s0 : p.w0, *w1 = sh ? p.s1 : p.w1;
     // this lane's weight row; block 0's words start loading, block 1's after
     // the first activations
     const uint32_t wcol = Q3 ? rt * PF_GU_R + 16u * wave + (col & 15u) : rt * PF_DN_R + 32u * wave + col;
-    const uint8_t *wrow = (Q3 && col >= 16u ? p.w1 : p.w0) +
+    const uint8_t *wrow = (Q3 && col >= 16u ? w1 : w0) +
                           ((uint64_t)e * p.out_rows + wcol) * ((uint64_t)nblk * (Q3 ? SF37_Q3_BYTES : SF37_Q2_BYTES));
     pf_raw_t<Q3, false> even;
     pf_raw_t<Q3, true> oddr;
@@ -689,12 +694,12 @@ __global__ void __launch_bounds__(PF_NW * 64, 2) pf_expert_kernel(pf_params p) {
         issue_act(0, 1);
         if (nblk > 1u) pf_wload<Q3, true>(oddr, wrow, 1u, kh);
         pf_loop<Q3, 1>(wrow, nblk, issue_act, s_act, s_gs, s_d, kh, col, even, oddr, acc);
-        pf_epilogue<Q3, 1>(p, acc, s_pair, s_w, s_tab, kh, col, wcol, cnt);
+        pf_epilogue<Q3, 1>(p, sh ? p.sh_clamp : p.clamp, acc, s_pair, s_w, s_tab, kh, col, wcol, cnt);
     } else {
         issue_act(0, 2);
         if (nblk > 1u) pf_wload<Q3, true>(oddr, wrow, 1u, kh);
         pf_loop<Q3, 2>(wrow, nblk, issue_act, s_act, s_gs, s_d, kh, col, even, oddr, acc);
-        pf_epilogue<Q3, 2>(p, acc, s_pair, s_w, s_tab, kh, col, wcol, cnt);
+        pf_epilogue<Q3, 2>(p, sh ? p.sh_clamp : p.clamp, acc, s_pair, s_w, s_tab, kh, col, wcol, cnt);
     }
 }
 
@@ -1122,8 +1127,12 @@ extern "C" int sf37k_pf_gate_up(float *mid, float *gate_out, float *up_out, cons
                                 const uint8_t *up_w, const void *act, const uint32_t *tiles,
                                 const uint32_t *sorted_pairs, const float *weights, uint32_t max_tiles,
                                 uint32_t n_tok, uint32_t topk, uint32_t in_dim, uint32_t mid_dim, float clamp,
-                                sf37_stream_t s) {
+                                const sf37_pf_shared *sh, sf37_stream_t s) {
     pf_params p = {};
+    p.s0 = sh ? sh->gate : NULL;
+    p.s1 = sh ? sh->up : NULL;
+    p.sh_id = sh ? sh->id : 0xffffffffu;
+    p.sh_clamp = sh ? sh->clamp : 0.0f;
     p.mid = mid;
     p.gate_out = gate_out;
     p.up_out = up_out;
@@ -1143,8 +1152,10 @@ extern "C" int sf37k_pf_gate_up(float *mid, float *gate_out, float *up_out, cons
 
 extern "C" int sf37k_pf_down(float *down_pair, const uint8_t *down_w, const void *act, const uint32_t *tiles,
                              const uint32_t *sorted_pairs, uint32_t max_tiles, uint32_t n_pairs, uint32_t mid_dim,
-                             uint32_t out_dim, sf37_stream_t s) {
+                             uint32_t out_dim, const sf37_pf_shared *sh, sf37_stream_t s) {
     pf_params p = {};
+    p.s0 = sh ? sh->down : NULL;
+    p.sh_id = sh ? sh->id : 0xffffffffu;
     p.down_pair = down_pair;
     p.w0 = down_w;
     pf_act_params(p, act, mid_dim, n_pairs);

@@ -1077,6 +1077,7 @@ typedef struct {
     const float *comb_base;   /* combine: out = comb_base + sum (may be out) */
     float *comb_resid;        /* combine: comb_resid += comb_base + sum instead */
     hipEvent_t comb_wait;     /* the combine waits for it (comb_base made on another stream) */
+    const sf37_pf_shared *sh; /* matrix-core path: an expert with tensors of its own */
 } routed_args;
 
 /* The combine of a routed pipeline, after the work comb_base waits for. */
@@ -1189,12 +1190,12 @@ static int routed_pf(const routed_args *a, const routed_scratch *s, float *out, 
            LAUNCH(SF37_HIP_STAGE_PF_TILES, sf37k_pf_tiles(s->tiles, s->ginfo, groups, st), "routed_moe tiles launch") &&
            LAUNCH(SF37_HIP_STAGE_PF_GATE_UP, sf37k_pf_gate_up(mid, gate_out, up_out, a->gate_w, a->up_w, s->xact,
                                                              s->tiles, s->sorted, a->weights, max_tiles, a->n_tok,
-                                                             a->topk, a->in_dim, a->mid_dim, a->clamp, st),
+                                                             a->topk, a->in_dim, a->mid_dim, a->clamp, a->sh, st),
                   "routed_moe mfma gate/up launch") &&
            LAUNCH(SF37_HIP_STAGE_PF_ACT_MID, sf37k_pf_act(0, s->mact, mid, a->mid_dim, pairs, st),
                   "routed_moe mfma mid codes launch") &&
            LAUNCH(SF37_HIP_STAGE_PF_DOWN, sf37k_pf_down(down_pair, a->down_w, s->mact, s->tiles, s->sorted, max_tiles,
-                                                       pairs, a->mid_dim, a->out_dim, st),
+                                                       pairs, a->mid_dim, a->out_dim, a->sh, st),
                   "routed_moe mfma down launch") &&
            routed_combine(a, out, down_pair);
 }
@@ -1523,7 +1524,7 @@ int sf37_hip_routed_moe_one(sf37_hip_tensor *out, sf37_hip_tensor *gate, sf37_hi
     if (moe_gate->bytes < gb || moe_up->bytes < gb || moe_down->bytes < db) return 0;
     routed_args a = {(const uint8_t *)moe_gate->ptr, (const uint8_t *)moe_up->ptr, (const uint8_t *)moe_down->ptr,
                      (const int32_t *)selected->ptr, (const float *)weights->ptr, n_total_expert, topk, in_dim,
-                     expert_mid_dim, out_dim, clamp, (const float *)x->ptr, 1, NULL, NULL, NULL};
+                     expert_mid_dim, out_dim, clamp, (const float *)x->ptr, 1, NULL, NULL, NULL, NULL};
     return routed_one_impl(out, gate, up, mid, down, &a);
 }
 
@@ -1553,7 +1554,7 @@ int sf37_hip_routed_moe_one_mapped(sf37_hip_tensor *out, sf37_hip_tensor *gate, 
                               expert_mid_dim, out_dim, x, 1))
         return 0;
     routed_args a = {NULL, NULL, NULL, (const int32_t *)selected->ptr, (const float *)weights->ptr, n_total_expert,
-                     topk, in_dim, expert_mid_dim, out_dim, clamp, (const float *)x->ptr, 1, NULL, NULL, NULL};
+                     topk, in_dim, expert_mid_dim, out_dim, clamp, (const float *)x->ptr, 1, NULL, NULL, NULL, NULL};
     if (!resolve_experts(model_map, model_size, gate_offset, up_offset, down_offset, n_total_expert, in_dim,
                          expert_mid_dim, out_dim, &a.gate_w, &a.up_w, &a.down_w))
         return 0;
@@ -1572,7 +1573,7 @@ int sf37_hip_routed_moe_batch_mapped(sf37_hip_tensor *out, sf37_hip_tensor *gate
                               expert_mid_dim, out_dim, x, n_tok))
         return 0;
     routed_args a = {NULL, NULL, NULL, (const int32_t *)selected->ptr, (const float *)weights->ptr, n_total_expert,
-                     topk, in_dim, expert_mid_dim, out_dim, clamp, (const float *)x->ptr, n_tok, NULL, NULL, NULL};
+                     topk, in_dim, expert_mid_dim, out_dim, clamp, (const float *)x->ptr, n_tok, NULL, NULL, NULL, NULL};
     if (!resolve_experts(model_map, model_size, gate_offset, up_offset, down_offset, n_total_expert, in_dim,
                          expert_mid_dim, out_dim, &a.gate_w, &a.up_w, &a.down_w))
         return 0;
@@ -1777,7 +1778,7 @@ static int layer_shared_q3q2(float *out, const sf37_hip_moe_layer_weights *w, co
     float *wts = (float *)(sw + align256((uint64_t)n_tok * 4u));
     routed_args a = {(const uint8_t *)w->sh_gate->ptr, (const uint8_t *)w->sh_up->ptr,
                      (const uint8_t *)w->sh_down->ptr, sel, wts, 1u, 1u, D, F, D, w->clamp_shared, x, n_tok, NULL, NULL,
-                     NULL};
+                     NULL, NULL};
     const int dec = decode_eligible(&a, 0);
     dec_extra ex;
     memset(&ex, 0, sizeof(ex));
@@ -1885,7 +1886,7 @@ static int moe_layer_impl(sf37_hip_tensor *out, sf37_hip_tensor *selected, sf37_
     }
     const sf37_stream_t st = (sf37_stream_t)g_stream;
     routed_args a = {(const uint8_t *)w->gate->ptr, (const uint8_t *)w->up->ptr, (const uint8_t *)w->down->ptr, NULL,
-                     NULL, E, K, D, F, D, w->clamp_routed, (const float *)x->ptr, n_tok, NULL, NULL, NULL};
+                     NULL, E, K, D, F, D, w->clamp_routed, (const float *)x->ptr, n_tok, NULL, NULL, NULL, NULL};
     const int fused = decode_eligible(&a, SF37_DEC_SELECT | (shared_q3 ? 0u : SF37_DEC_SHARED));
     /* a Q3GU/Q2D shared expert as one more slot inside the routed decode
      * launches (its pairs grouped two at a time, so its up and down items
@@ -1981,6 +1982,34 @@ static int moe_layer_impl(sf37_hip_tensor *out, sf37_hip_tensor *selected, sf37_
                                        (const float *)w->router_bias->ptr, E, K, w->scale, n_tok, st),
                    "moe_layer router_select launch"))
         return 0;
+    /* a Q3GU/Q2D shared expert as one more expert (id E, weight 1, its own
+     * tensors) in one more slot of every token inside the routed matrix-core
+     * launches: by itself it is one group whose tiles fill a fraction of the
+     * chip (187 tokens: 907 us on the dot kernels, which groups under
+     * prefill_min_pairs pairs take).  The combine's slot-order sum adds its
+     * row last, the same single rounding as shared + (slots 0..K-1). */
+    if (shared_q3 && E + 1u <= DISPATCH_MAX_EXPERTS) {
+        const sf37_pf_shared shp = {(const uint8_t *)w->sh_gate->ptr, (const uint8_t *)w->sh_up->ptr,
+                                    (const uint8_t *)w->sh_down->ptr, E, w->clamp_shared};
+        const uint64_t slots = align256((uint64_t)n_tok * (K + 1u) * 4u);
+        routed_args p9 = a;
+        p9.n_expert = E + 1u;
+        p9.topk = K + 1u;
+        if (prefill_eligible(&p9, 0) && aligned4(shp.gate) && aligned4(shp.up) && aligned4(shp.down)) {
+            char *buf = (char *)layer_buf(10, 2u * slots);
+            if (!buf) return 0;
+            int32_t *sel9 = (int32_t *)buf;
+            float *wts9 = (float *)(buf + slots);
+            if (!LAUNCH(SF37_HIP_STAGE_SELECT, sf37k_moe_append_shared(sel9, wts9, sel, wts, K, E, n_tok, st),
+                        "moe_layer shared slot launch"))
+                return 0;
+            p9.selected = sel9;
+            p9.weights = wts9;
+            p9.sh = &shp;
+            p9.comb_resid = resid;
+            return routed_q8k(&p9, (float *)out->ptr, NULL, NULL, NULL, NULL, 0);
+        }
+    }
     /* shared expert into out: Q3GU/Q2D on the Q8_K path, or Q8_0 gate/up
      * pair -> SwiGLU -> Q8_0 down */
     if (shared_q3) {
@@ -2049,7 +2078,7 @@ int sf37_hip_moe_layer_noalloc(sf37_hip_tensor *out, sf37_hip_tensor *selected, 
     const int run_router = !logits_in || (g_opt_router_always && w->router);
     if (!layer_weights_ok(w, run_router)) return 0;
     routed_args a = {(const uint8_t *)w->gate->ptr, (const uint8_t *)w->up->ptr, (const uint8_t *)w->down->ptr, NULL,
-                     NULL, E, K, D, F, D, w->clamp_routed, (const float *)x->ptr, n_tok, NULL, NULL, NULL};
+                     NULL, E, K, D, F, D, w->clamp_routed, (const float *)x->ptr, n_tok, NULL, NULL, NULL, NULL};
     if ((run_router && w->router_type != SF37_HIP_TYPE_F32) || w->shared_type == SF37_HIP_TYPE_Q3GU ||
         !decode_eligible(&a, SF37_DEC_SELECT | SF37_DEC_SHARED)) {
         fprintf(stderr, "sf37: HIP moe_layer_noalloc takes decode batches of 1..%u tokens on the Q8_K path with an "

@@ -80,7 +80,7 @@ int sf37k_moe_down(float *down_pair, const uint8_t *down_w, const void *midq,
                    uint32_t max_groups, uint32_t max_group_pairs, uint32_t mid_dim,
                    uint32_t out_dim, sf37_stream_t s);
 /* Slot-order sum of the per-pair rows: out = [base +] sum (base may be out);
- * with resid, resid = resid + (base + sum) instead and out is not written. */
+ * with resid, resid = resid + ([base +] sum) instead and out is not written. */
 int sf37k_moe_combine(float *out, const float *down_pair, const float *base, float *resid, uint32_t topk,
                       uint32_t out_dim, uint32_t n_tok, sf37_stream_t s);
 /* Build the groups from selected experts: stable counting sort of pairs by
@@ -92,6 +92,10 @@ uint64_t sf37k_moe_dispatch_scratch_bytes(uint32_t n_pairs, uint32_t n_expert);
 int sf37k_moe_dispatch(uint32_t *group_info, uint32_t *sorted_pairs, uint32_t *counts,
                        uint32_t *offsets, const int32_t *selected, uint32_t n_pairs,
                        uint32_t n_expert, uint32_t *hist, sf37_stream_t s);
+/* Selections and weights with one more slot per token: id n_expert, weight 1
+ * (a shared expert in the routed formats run as one more expert). */
+int sf37k_moe_append_shared(int32_t *sel_out, float *w_out, const int32_t *sel, const float *w, uint32_t topk,
+                            uint32_t n_expert, uint32_t n_tok, sf37_stream_t s);
 /* One group per slot for a single token (no sort), as routed_moe_one. */
 int sf37k_moe_slots(uint32_t *group_info, uint32_t *sorted_pairs, const int32_t *selected,
                     uint32_t topk, uint32_t n_expert, sf37_stream_t s);
@@ -127,14 +131,21 @@ int sf37k_pf_supported(uint32_t in_dim, uint32_t mid_dim, uint32_t out_dim);
 uint64_t sf37k_pf_act_bytes(uint32_t dim, uint64_t n_rows);
 int sf37k_pf_act(int q3, void *act, const float *x, uint32_t dim, uint32_t n_rows, sf37_stream_t s);
 int sf37k_pf_tiles(uint32_t *tiles, const uint32_t *group_info, uint32_t max_groups, sf37_stream_t s);
+/* An expert whose weights are tensors of their own: the group of expert id
+ * `id` reads these (and the SwiGLU takes this clamp).  NULL for none. */
+typedef struct {
+    const uint8_t *gate, *up, *down;
+    uint32_t id;
+    float clamp;
+} sf37_pf_shared;
 int sf37k_pf_gate_up(float *mid, float *gate_out, float *up_out, const uint8_t *gate_w,
                      const uint8_t *up_w, const void *act, const uint32_t *tiles,
                      const uint32_t *sorted_pairs, const float *weights, uint32_t max_tiles,
                      uint32_t n_tok, uint32_t topk, uint32_t in_dim, uint32_t mid_dim, float clamp,
-                     sf37_stream_t s);
+                     const sf37_pf_shared *sh, sf37_stream_t s);
 int sf37k_pf_down(float *down_pair, const uint8_t *down_w, const void *act, const uint32_t *tiles,
                   const uint32_t *sorted_pairs, uint32_t max_tiles, uint32_t n_pairs, uint32_t mid_dim,
-                  uint32_t out_dim, sf37_stream_t s);
+                  uint32_t out_dim, const sf37_pf_shared *sh, sf37_stream_t s);
 
 /* Shared expert (Q8_0) on the int8 matrix cores for many tokens
  * (k_prefill.hip): Q8_0 activations (a8: n_tok x dim int8 codes, xs: n_tok x
