@@ -221,11 +221,12 @@ __global__ void __launch_bounds__(256) f32_matvec_kernel(float *__restrict__ out
     }
 }
 
+template <int S>
 __global__ void __launch_bounds__(256) router_select_kernel(int32_t *__restrict__ selected,
                                                             float *__restrict__ weights,
                                                             float *__restrict__ probs,
                                                             const float *__restrict__ logits,
-                                                            const double *__restrict__ part, uint32_t S,
+                                                            const double *__restrict__ part,
                                                             const float *__restrict__ bias,
                                                             uint32_t n_experts, uint32_t topk,
                                                             float scale, uint32_t n_tok) {
@@ -237,16 +238,24 @@ __global__ void __launch_bounds__(256) router_select_kernel(int32_t *__restrict_
     int32_t *so[1] = {selected + (uint64_t)t * topk};
     float *wo[1] = {weights + (uint64_t)t * topk};
     float *po[1] = {probs ? probs + (uint64_t)t * n_experts : nullptr};
-    if (part) {
+    if constexpr (S > 1) {
         // logits left as S binary64 slices by the split router GEMM: added in
-        // slice order and rounded once, as rl_reduce_kernel does
+        // slice order and rounded once, as rl_reduce_kernel does.  All of a
+        // logit's slices are loaded before the first add: with few tokens
+        // (few waves) the loads' latencies are what the launch takes, one
+        // after the other 28 us at 21 tokens and 16 slices, in flight
+        // together 10 us.
         const uint64_t n = (uint64_t)n_tok * n_experts;
         const double *pt = part + (uint64_t)t * n_experts;
         sf37_wave_topk<1>(
-            [pt, n, S](uint32_t, uint32_t e) {
-                double v = pt[e];
-                for (uint32_t k = 1; k < S; k++) v += pt[(uint64_t)k * n + e];
-                return (float)v;
+            [pt, n](uint32_t, uint32_t e) {
+                double v[S];
+#pragma unroll
+                for (int k = 0; k < S; k++) v[k] = pt[(uint64_t)k * n + e];
+                double sum = v[0];
+#pragma unroll
+                for (int k = 1; k < S; k++) sum += v[k];
+                return (float)sum;
             },
             bias, n_experts, topk, scale, tab, so, wo, po);
     } else {
@@ -333,8 +342,18 @@ extern "C" int sf37k_router_select_part(int32_t *selected, float *weights, float
                                         const double *part, uint32_t slices, const float *bias, uint32_t n_experts,
                                         uint32_t topk, float scale, uint32_t n_tok, sf37_stream_t s) {
     if (n_tok == 0) return 0;
-    hipLaunchKernelGGL(router_select_kernel, dim3((n_tok + 3) / 4), dim3(256), 0, (hipStream_t)s, selected,
-                       weights, probs, logits, slices > 1u ? part : (const double *)NULL, slices, bias, n_experts,
-                       topk, scale, n_tok);
+#define SF37_SELECT(S)                                                                                             \
+    hipLaunchKernelGGL(router_select_kernel<S>, dim3((n_tok + 3) / 4), dim3(256), 0, (hipStream_t)s, selected,     \
+                       weights, probs, logits, part, bias, n_experts, topk, scale, n_tok)
+    switch (slices) {
+        case 0:
+        case 1: SF37_SELECT(1); break;
+        case 2: SF37_SELECT(2); break;
+        case 4: SF37_SELECT(4); break;
+        case 8: SF37_SELECT(8); break;
+        case 16: SF37_SELECT(16); break;
+        default: return (int)hipErrorInvalidValue;
+    }
+#undef SF37_SELECT
     return (int)hipGetLastError();
 }
