@@ -54,8 +54,13 @@ static int64_t g_opt_router_always = 0;
 static int64_t g_opt_up_dyn_pct = -1, g_opt_up_wgs = 0, g_opt_dn_wgs = 0, g_opt_upsel_max_tok = 1;
 static int64_t g_opt_down_combine = 1;
 static int64_t g_opt_prefill = 1;
-static int64_t g_opt_prefill_min_pairs = 256;
-static int64_t g_opt_shared_min_tok = 64;
+/* Batches past the fused decode sizes go to the matrix cores: measured per
+ * layer (us, staged / matrix cores with the shared expert on its stream) 17
+ * tokens 301 / 266, 21 348 / 302, 31 449 / 369, 24 tokens of Zipf routing 297
+ * / 123 (17 tokens x top-8 = 136 pairs).  The shared expert alone: 4096 -> 2 x
+ * 1280 and back at 17 tokens 56 us on the dot kernels, 47 us here. */
+static int64_t g_opt_prefill_min_pairs = 128;
+static int64_t g_opt_shared_min_tok = 17;
 static int64_t g_opt_q8_0_min_tok = 20;
 static int64_t g_opt_shared_stream = 1;
 static int64_t g_opt_shared_slot = 1;
