@@ -43,6 +43,7 @@
 #include <type_traits>
 
 #include "sf37_blocks.h"
+#include "sf37_dispatch.h"
 #include "sf37_launch.h"
 
 namespace {
@@ -113,21 +114,18 @@ constexpr int QUAD_XOR1 = 0xB1, QUAD_XOR2 = 0x4E;
 // Activation kernel: Q8_K of one (row, 256-block) per wave, the codes as
 // 6-bit fields, -gsum/64 of the four groups and d.
 // ---------------------------------------------------------------------------
+// A wave's units u0, u0 + stride, ..; row: PF_BLK bytes of LDS of its own.
 template <bool Q3>
-__global__ void __launch_bounds__(256) pf_act_kernel(uint32_t *__restrict__ codes, uint32_t *__restrict__ rec,
-                                                     const float *__restrict__ x, uint32_t nblk, uint32_t n_rows) {
-    // each wave owns its LDS row and walks the (row, block) units wave by
-    // wave over the grid; nothing is shared between waves
-    __shared__ __align__(16) uint8_t st[4][PF_BLK];
-    const uint32_t wv = threadIdx.x >> 6, lane = threadIdx.x & 63u;
-    const uint32_t units = nblk * n_rows, stride = gridDim.x * 4u;
-    uint8_t *row = st[wv];
+__device__ __forceinline__ void pf_act_units(uint32_t *__restrict__ codes, uint32_t *__restrict__ rec,
+                                             const float *__restrict__ x, uint32_t units, uint32_t u0,
+                                             uint32_t stride, uint8_t *row) {
+    const uint32_t lane = threadIdx.x & 63u;
     // the lane's half-group (48 bytes), its quad in it, its place in the quad
     const uint32_t hb = (lane >> 3) * 48u, quad = (lane >> 2) & 1u, qj = lane & 3u;
     // piece `lane` (lanes < 24) of the output from the half-group order
     const uint32_t pc = 4u * (lane >> 3) + ((lane & 7u) >> 1);
     const uint32_t piece = (2u * (pc / 3u) + (lane & 1u)) * 48u + 16u * (pc % 3u);
-    for (uint32_t u = blockIdx.x * 4u + wv; u < units; u += stride) {
+    for (uint32_t u = u0; u < units; u += stride) {
         const float4 xv = *(const float4 *)(x + (uint64_t)u * SF37_QK + 4u * lane);
         const float v[4] = {xv.x, xv.y, xv.z, xv.w};
         int8_t q[4];
@@ -199,6 +197,42 @@ __global__ void __launch_bounds__(256) pf_act_kernel(uint32_t *__restrict__ code
         }
         if (lane == 0u) rec[(uint64_t)u * (PF_REC / 4u) + 4u] = __builtin_bit_cast(uint32_t, d);
     }
+}
+
+// Each wave owns its LDS row and walks the (row, block) units wave by wave
+// over the grid; nothing is shared between waves.
+template <bool Q3>
+__global__ void __launch_bounds__(256) pf_act_kernel(uint32_t *__restrict__ codes, uint32_t *__restrict__ rec,
+                                                     const float *__restrict__ x, uint32_t nblk, uint32_t n_rows) {
+    __shared__ __align__(16) uint8_t st[4][PF_BLK];
+    const uint32_t wv = threadIdx.x >> 6;
+    pf_act_units<Q3>(codes, rec, x, nblk * n_rows, blockIdx.x * 4u + wv, gridDim.x * 4u, st[wv]);
+}
+
+// What the gate/up launch of a small batch needs, in one launch: workgroup 0
+// sorts the pairs by expert and lists the tiles, the others write the rows'
+// operands.  Each of the three is latency-bound, about 5 us with its launch.
+// Measured per layer, three launches / one: 21 tokens 265 / 258 us, 64 tokens
+// 155 / 150, 187 tokens 530 / 523.  At 512 tokens (4096 pairs) 370 / 375: the
+// 1024-thread workgroups then wait for whole CUs that the shared expert's
+// GEMM holds on its stream, which the 256-thread ones of pf_act_kernel do
+// not, so the line is at PF_START_PAIRS pairs.
+constexpr uint32_t PF_START_PAIRS = 2048;
+static_assert(PF_START_PAIRS <= DISP_ONE_PAIRS, "one workgroup sorts them");
+__global__ void __launch_bounds__(1024) pf_start_kernel(uint32_t *__restrict__ codes, uint32_t *__restrict__ rec,
+                                                        const float *__restrict__ x, uint32_t units,
+                                                        uint32_t *__restrict__ group_info,
+                                                        uint32_t *__restrict__ sorted, uint32_t *__restrict__ counts,
+                                                        uint32_t *__restrict__ offsets, uint32_t *__restrict__ tiles,
+                                                        const int32_t *__restrict__ selected, uint32_t n_pairs,
+                                                        uint32_t n_expert) {
+    __shared__ __align__(16) uint8_t st[16][PF_BLK];
+    if (blockIdx.x == 0u) {
+        dispatch_pairs<PF_T>(group_info, sorted, counts, offsets, tiles, selected, n_pairs, n_expert);
+        return;
+    }
+    const uint32_t wv = threadIdx.x >> 6;
+    pf_act_units<true>(codes, rec, x, units, (blockIdx.x - 1u) * 16u + wv, (gridDim.x - 1u) * 16u, st[wv]);
 }
 
 // ---------------------------------------------------------------------------
@@ -1108,6 +1142,24 @@ extern "C" int sf37k_pf_act(int q3, void *act, const float *x, uint32_t dim, uin
         hipLaunchKernelGGL(pf_act_kernel<true>, grid, dim3(256), 0, (hipStream_t)s, codes, rec, x, nblk, n_rows);
     else
         hipLaunchKernelGGL(pf_act_kernel<false>, grid, dim3(256), 0, (hipStream_t)s, codes, rec, x, nblk, n_rows);
+    return (int)hipGetLastError();
+}
+
+extern "C" int sf37k_pf_start_supported(uint32_t n_pairs, uint32_t n_expert) {
+    return n_pairs > 0 && n_pairs <= PF_START_PAIRS && n_expert > 0 && n_expert <= DISP_MAX_E;
+}
+
+extern "C" int sf37k_pf_start(void *act, const float *x, uint32_t dim, uint32_t n_rows, uint32_t *group_info,
+                              uint32_t *sorted_pairs, uint32_t *counts, uint32_t *offsets, uint32_t *tiles,
+                              const int32_t *selected, uint32_t n_pairs, uint32_t n_expert, sf37_stream_t s) {
+    const uint32_t nblk = dim / SF37_QK;
+    const uint64_t units = (uint64_t)nblk * n_rows;
+    if (units > 0xffffffffu || !sf37k_pf_start_supported(n_pairs, n_expert)) return (int)hipErrorInvalidValue;
+    // sixteen units per workgroup pass; at most two workgroups per CU of them
+    const uint64_t wgs = (units + 15u) / 16u;
+    hipLaunchKernelGGL(pf_start_kernel, dim3(1u + (unsigned)(wgs < 512u ? wgs : 512u)), dim3(1024), 0, (hipStream_t)s,
+                       (uint32_t *)act, (uint32_t *)pf_act_rec(act, nblk, n_rows), x, (uint32_t)units, group_info,
+                       sorted_pairs, counts, offsets, tiles, selected, n_pairs, n_expert);
     return (int)hipGetLastError();
 }
 

@@ -1187,13 +1187,21 @@ static int routed_pf(const routed_args *a, const routed_scratch *s, float *out, 
     const uint32_t pairs = a->n_tok * a->topk;
     const uint32_t groups = a->n_expert;
     const uint32_t max_tiles = sf37k_pf_max_tiles(pairs, groups);
-    return LAUNCH(SF37_HIP_STAGE_PF_ACT_X, sf37k_pf_act(1, s->xact, a->x, a->in_dim, a->n_tok, st),
-                  "routed_moe mfma input codes launch") &&
-           LAUNCH(SF37_HIP_STAGE_DISPATCH, sf37k_moe_dispatch(s->ginfo, s->sorted, s->counts, s->offsets, a->selected,
-                                                              pairs, a->n_expert, s->hist, st),
-                  "routed_moe dispatch launch") &&
-           LAUNCH(SF37_HIP_STAGE_PF_TILES, sf37k_pf_tiles(s->tiles, s->ginfo, groups, st), "routed_moe tiles launch") &&
-           LAUNCH(SF37_HIP_STAGE_PF_GATE_UP, sf37k_pf_gate_up(mid, gate_out, up_out, a->gate_w, a->up_w, s->xact,
+    if (sf37k_pf_start_supported(pairs, groups)) {
+        if (!LAUNCH(SF37_HIP_STAGE_DISPATCH, sf37k_pf_start(s->xact, a->x, a->in_dim, a->n_tok, s->ginfo, s->sorted,
+                                                            s->counts, s->offsets, s->tiles, a->selected, pairs,
+                                                            a->n_expert, st),
+                    "routed_moe dispatch and input codes launch"))
+            return 0;
+    } else if (!(LAUNCH(SF37_HIP_STAGE_PF_ACT_X, sf37k_pf_act(1, s->xact, a->x, a->in_dim, a->n_tok, st),
+                        "routed_moe mfma input codes launch") &&
+                 LAUNCH(SF37_HIP_STAGE_DISPATCH, sf37k_moe_dispatch(s->ginfo, s->sorted, s->counts, s->offsets,
+                                                                    a->selected, pairs, a->n_expert, s->hist, st),
+                        "routed_moe dispatch launch") &&
+                 LAUNCH(SF37_HIP_STAGE_PF_TILES, sf37k_pf_tiles(s->tiles, s->ginfo, groups, st),
+                        "routed_moe tiles launch")))
+        return 0;
+    return LAUNCH(SF37_HIP_STAGE_PF_GATE_UP, sf37k_pf_gate_up(mid, gate_out, up_out, a->gate_w, a->up_w, s->xact,
                                                              s->tiles, s->sorted, a->weights, max_tiles, a->n_tok,
                                                              a->topk, a->in_dim, a->mid_dim, a->clamp, a->sh, st),
                   "routed_moe mfma gate/up launch") &&

@@ -130,6 +130,12 @@ uint32_t sf37k_pf_max_tiles(uint32_t n_pairs, uint32_t max_groups);
 int sf37k_pf_supported(uint32_t in_dim, uint32_t mid_dim, uint32_t out_dim);
 uint64_t sf37k_pf_act_bytes(uint32_t dim, uint64_t n_rows);
 int sf37k_pf_act(int q3, void *act, const float *x, uint32_t dim, uint32_t n_rows, sf37_stream_t s);
+/* pf_act(q3 = 1), the dispatch and the tiles in one launch, for small
+ * batches. */
+int sf37k_pf_start_supported(uint32_t n_pairs, uint32_t n_expert);
+int sf37k_pf_start(void *act, const float *x, uint32_t dim, uint32_t n_rows, uint32_t *group_info,
+                   uint32_t *sorted_pairs, uint32_t *counts, uint32_t *offsets, uint32_t *tiles,
+                   const int32_t *selected, uint32_t n_pairs, uint32_t n_expert, sf37_stream_t s);
 int sf37k_pf_tiles(uint32_t *tiles, const uint32_t *group_info, uint32_t max_groups, sf37_stream_t s);
 /* An expert whose weights are tensors of their own: the group of expert id
  * `id` reads these (and the SwiGLU takes this clamp).  NULL for none. */
