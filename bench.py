@@ -538,13 +538,13 @@ def prefill_bench(args, H, layer, config):
     counts = np.bincount(sel.read(np.int32).ravel(), minlength=E)
     # VALU issue the exact arithmetic needs at least (the matrix-core kernels'
     # bound): per padded pair, output and 256-block the canonical epilogue's 5
-    # operations; per tile the weights' dequantisation (1.5 operations per Q3
-    # code, 1 per Q2 code); at 16 lanes per cycle per SIMD, 1024 SIMDs, 2.4 GHz
+    # operations; per tile the weights' dequantisation (about 0.33 operations
+    # per Q3 code, 0.38 per Q2 code); at 16 lanes per cycle per SIMD, 1024 SIMDs, 2.4 GHz
     tiles = [min(64, c - 64 * i) for c in counts for i in range((int(c) + 63) // 64)]
     padded = sum(32 * ((t + 31) // 32) for t in tiles)
     nbk, nbf = K // 256, F // 256
-    valu = {"pf_gate_up": padded * 2 * F * nbk * 5 + len(tiles) * 2 * F * K * 1.5,
-            "pf_down": padded * K * nbf * 5 + len(tiles) * K * F * 1.0}
+    valu = {"pf_gate_up": padded * 2 * F * nbk * 5 + len(tiles) * 2 * F * K * 0.33,
+            "pf_down": padded * K * nbf * 5 + len(tiles) * K * F * 0.38}
     lane_ops_per_s = 1024 * 16 * 2.4e9
     for k, v in valu.items():
         ceil_ms = v / lane_ops_per_s * 1e3
@@ -556,7 +556,8 @@ def prefill_bench(args, H, layer, config):
             "tokens_per_s_per_layer": round(n_tok / (ms * 1e-3), 1),
             "routed_mfma": {"bound": "mfma", "achieved": round(routed_t, 1), "peak": MFMA_F16_PEAK_TFLOPS,
                             "unit": "TFLOP/s", "frac": round(routed_t / MFMA_F16_PEAK_TFLOPS, 4),
-                            "dtype": "f16 operands holding exact small integers, fp32 accumulate",
+                            "dtype": "6-bit float operands (E2M3, E3M2) holding exact small integers, "
+                                     "fp32 accumulate; peak: bf16 dense",
                             "timing": "HIP events around each launch on its stream (include the dispatch; "
                                       "profiles/prefill_layer_kernel_trace.md has rocprofv3 kernel durations)"},
             "kernels": mfma, "max_pairs_per_expert": int(counts.max()), "idle_experts": int((counts == 0).sum()),
